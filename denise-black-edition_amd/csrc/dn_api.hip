@@ -162,7 +162,7 @@ int build_lists(dn_ctx *c)
     };
     std::vector<Item> lists[4];
     // lists 0 and 2 belong to the velocity sweep, 1 and 3 to the stress sweep
-    auto add = [&](int which, int i, int j, int kind, int idx) {
+    auto add_tile = [&](int which, int i, int j, int kind, int idx) {
         const Tile &t = (which == 0 || which == 2) ? c->tile_v : c->tile_s;
         const int ntx = (which == 0 || which == 2) ? c->ntx_v : c->ntx_s;
         const int tx = (i - 1) / t.width(), ty = (j - 1) / t.rows();
@@ -173,6 +173,14 @@ int build_lists(dn_ctx *c)
         it.e.kind = kind;
         it.e.idx = idx;
         lists[which].push_back(it);
+    };
+    struct Point {
+        int which, i, j, kind, idx;
+    };
+    std::vector<Point> points;
+    auto add = [&](int which, int i, int j, int kind, int idx) {
+        add_tile(which, i, j, kind, idx);
+        if (c->res.ok) points.push_back(Point{which, i, j, kind, idx});
     };
     const int ns = (int)c->src_ix.size(), nr = (int)c->rec_ix.size();
     const int seismo = c->p.seismo;
@@ -257,6 +265,51 @@ int build_lists(dn_ctx *c)
         HIP_OK(h2d(c->stream, c->lst_off[w], off.data(), off.size() * sizeof(int)));
         HIP_OK(h2d(c->stream, c->lst_ent[w], ent.data(), ent.size() * sizeof(Ent)));
     }
+    if (!c->res.ok) return DN_OK;
+    // the same points by tile and owner thread of the chip-resident loop
+    const ResPlan &pl = c->res;
+    const int HP = 4 * ((c->fdoh + 3) / 4), LP = res_width(pl.ry) + 2 * HP;
+    std::vector<int> blk;
+    for (int w = 0; w < 4; ++w) {
+        struct Own {
+            int tile, own, el, kind, idx;
+        };
+        std::vector<Own> v;
+        c->res_lst_ok[w] = true;
+        for (const Point &q : points) {
+            if (q.which != w) continue;
+            // the surface condition of row 1 follows the sources added there
+            if (q.j == 1 && c->a.mirror && (q.kind == E_EXPLOSIVE || q.kind == E_ADJ_P)) c->res_lst_ok[w] = false;
+            const int bx = (q.i - 1) / pl.tw, by = (q.j - 1) / pl.th;
+            const int x = q.i - 1 - bx * pl.tw, y = q.j - 1 - by * pl.th;
+            v.push_back(Own{by * pl.gx + bx, y / pl.ry * pl.nthx + x / pl.vx, (y + c->fdoh) * LP + HP + x, q.kind, q.idx});
+        }
+        std::stable_sort(v.begin(), v.end(), [](const Own &x, const Own &y) {
+            return x.tile < y.tile || (x.tile == y.tile && x.own < y.own);
+        });
+        std::vector<int> off((size_t)pl.tiles() + 1, 0);
+        for (const Own &o : v) off[(size_t)o.tile + 1]++;
+        c->res_most[w] = 0;
+        for (int k = 0; k < pl.tiles(); ++k) {
+            c->res_most[w] = std::max(c->res_most[w], off[(size_t)k + 1]);
+            off[(size_t)k + 1] += off[k];
+        }
+        c->res_off[w] = blk.size();
+        blk.insert(blk.end(), off.begin(), off.end());
+        c->res_own[w] = blk.size();
+        for (const Own &o : v) blk.push_back(o.own);
+        blk.resize((blk.size() + 1) / 2 * 2);  // entries are pairs
+        c->res_ent[w] = blk.size();
+        for (const Own &o : v) {
+            blk.push_back(o.kind << 24 | o.el);
+            blk.push_back(o.idx);
+        }
+    }
+    if (c->res_lst) c->dfree(c->res_lst);
+    c->res_lst = nullptr;
+    int rc;
+    if ((rc = c->dalloc((void **)&c->res_lst, blk.size() * sizeof(int)))) return rc;
+    HIP_OK(h2d(c->stream, c->res_lst, blk.data(), blk.size() * sizeof(int)));
     return DN_OK;
 }
 
@@ -349,7 +402,7 @@ int dn::zero_state(dn_ctx *c)
     }
     const size_t nxb = (size_t)c->p.ny * 2 * c->p.fw, nyb = (size_t)2 * c->p.fw * c->p.nx;
     for (int k = 0; k < 9; ++k) HIP_OK(hipMemsetAsync(c->psi[k], 0, (k < 5 ? nxb : nyb) * sizeof(float) + 4, c->stream));
-    HIP_OK(hipMemsetAsync(c->acq.nan_step, 0, sizeof(int), c->stream));
+    HIP_OK(hipMemsetAsync(c->acq.nan_step, 0, 2 * sizeof(int), c->stream));
     return DN_OK;
 }
 
@@ -365,7 +418,9 @@ hipEvent_t pool_event(dn_ctx *c, size_t k)
     return c->pool[k];
 }
 
-int finish_run(dn_ctx *c, size_t nsample_events)
+// aborted (chip-resident runs): set when the workgroups gave up waiting for
+// each other and left; the run then has no result
+int finish_run(dn_ctx *c, size_t nsample_events, bool *aborted = nullptr)
 {
     HIP_OK(hipEventRecord(c->ev1, c->stream));
     HIP_OK(hipStreamSynchronize(c->stream));
@@ -386,10 +441,97 @@ int finish_run(dn_ctx *c, size_t nsample_events)
         c->v_ms /= c->samples;
         c->s_ms /= c->samples;
     }
-    int nan_step = 0;
-    HIP_OK(d2h(c->stream, &nan_step, c->acq.nan_step, sizeof(int)));
-    if (nan_step)
-        return fail(DN_ERR_UNSTABLE, " Simulation is unstable ! (NaN at time step " + std::to_string(nan_step) + ")");
+    int word[2] = {0, 0};  // NaN step, abort
+    HIP_OK(d2h(c->stream, word, c->acq.nan_step, sizeof word));
+    if (word[1] && aborted) {
+        *aborted = true;
+        return DN_OK;
+    }
+    if (word[0])
+        return fail(DN_ERR_UNSTABLE, " Simulation is unstable ! (NaN at time step " + std::to_string(word[0]) + ")");
+    return DN_OK;
+}
+
+// LDS of a run: the plan's, and the point lists (16-byte rounded)
+size_t res_lds(const dn_ctx *c, int sw)
+{
+    return c->res.lds + (size_t)((c->res_most[2 * sw] + c->res_most[2 * sw + 1] + 1) & ~1) * sizeof(uint2);
+}
+
+// Runs that the chip-resident loop takes: the grid fits (res_plan), a kernel
+// is compiled for the physics, and nothing in the run belongs to the host
+// loop or to a sweep's own launch: no moment-tensor source (its increments
+// land between launches), no CPML stretching (k_max_PML 1), no ux / uy / uxy output (GRAD_FORM 2 with
+// snapshots), no energy sums, wavefield snapshots or kernel sampling, and no
+// sweep shape or cache policy chosen by the caller.
+bool res_applies(const dn_ctx *c, int sw)
+{
+    if (!c->res.ok || c->sweeps_chosen || !res_compiled(c->a.physics, c->p.L, sw)) return false;
+    if (!c->res_lst_ok[2 * sw] || !c->res_lst_ok[2 * sw + 1]) return false;
+    if (c->res_most[2 * sw] > RES_ENT || c->res_most[2 * sw + 1] > RES_ENT) return false;
+    if (res_lds(c, sw) > res_pool_lds(c->res_pool)) return false;
+    if (c->qtype == 5 || c->eprecond || c->snap_fn || c->sample_every > 0) return false;
+    if (c->p.mode > 0 && c->p.grad_form != 1) return false;
+    for (int k : {P_KX, P_KXH, P_KY, P_KYH})
+        for (int h = 1; h <= 2 * c->p.fw; ++h)
+            if (c->setup.pml[k][h] != 1.0f) return false;
+    // the division by DH assumes no range of its own, but 1 / DH must be normal
+    return c->p.dh >= 0x1p-60f && c->p.dh <= 0x1p60f;
+}
+
+// nsteps time steps from the zeroed state by the chip-resident loop.  *done
+// stays false when it did not run to its end (no free CUs, refused launch,
+// abandoned wait): the state is then undefined and the caller starts over.
+int res_run(dn_ctx *c, const StepCtl &ctl, int sw, int nsteps, bool *done)
+{
+    *done = false;
+    ResLease l;
+    ResPlan pl = c->res;
+    pl.lds = res_lds(c, sw);
+    if (!res_pool_take(c->res_pool, pl, nsteps, &l)) return DN_OK;
+    ResArgs r{};
+    r.tw = pl.tw;
+    r.th = pl.th;
+    r.nthx = pl.nthx;
+    r.gx = pl.gx;
+    r.gy = pl.gy;
+    r.ncomp = pl.ncomp;
+    r.nk_s = pl.nk_s;
+    r.nk_v = pl.nk_v;
+    r.cap = pl.cap;
+    r.ncx = pl.ncx;
+    r.ncy = pl.ncy;
+    r.nve = c->res_most[2 * sw];
+    r.nse = c->res_most[2 * sw + 1];
+    r.nlast = nsteps;
+    r.fwdstore = c->p.mode > 0;
+    r.dtinv = c->p.dtinv > 0 ? c->p.dtinv : 1;
+    r.vp1_form = c->p.grad_form == 1 || c->p.grad_form == 2;
+    r.vec = c->p.nx % 4 == 0;
+    r.rdh = 1.0 / (double)c->p.dh;
+    r.mbox = l.mbox;
+    r.abort = c->acq.nan_step + 1;
+    const int v = 2 * sw, s = 2 * sw + 1;
+    r.voff = c->res_lst + c->res_off[v];
+    r.vown = c->res_lst + c->res_own[v];
+    r.vent = reinterpret_cast<const uint2 *>(c->res_lst + c->res_ent[v]);
+    r.soff = c->res_lst + c->res_off[s];
+    r.sown = c->res_lst + c->res_own[s];
+    r.sent = reinterpret_cast<const uint2 *>(c->res_lst + c->res_ent[s]);
+    unsigned tag = l.tag0;
+    bool ok = true;
+    for (int n = 1; n <= nsteps && ok; n += RES_CHUNK) {
+        r.n0 = n;
+        r.n1 = std::min(n + RES_CHUNK - 1, nsteps);
+        r.tag0 = tag;
+        tag += (unsigned)(r.n1 - r.n0 + 2);
+        ok = res_launch(c->a, ctl, c->acq, r, pl, c->fdoh, sw, c->stream);
+    }
+    bool aborted = !ok;
+    const int rc = finish_run(c, 0, &aborted);
+    res_pool_give(c->res_pool, l);
+    if (rc) return rc;
+    *done = !aborted;
     return DN_OK;
 }
 
@@ -450,7 +592,7 @@ std::vector<size_t> plan_sizes(const dn_params &p, int nsrc, int ntr)
         add((size_t)p.nx * p.ny * ntd * sizeof(float), (size_t)snap_planes(p.physics));
         add((size_t)p.nx * p.ny * sizeof(float), 6);
     }
-    add(sizeof(int), 1);
+    add(2 * sizeof(int), 1);
     add(sizeof(double) * l2_scratch_doubles(), 1);
     if (nsrc > 0) {
         add(sizeof(int) * nsrc, 3);
@@ -608,10 +750,12 @@ static int ctx_create(const dn_params *p, int device, dn_arena *arena, dn_ctx **
         for (auto m : grads)
             if ((rc = c->dalloc((void **)m, g))) return bail(rc);
     }
-    if ((rc = c->dalloc((void **)&c->acq.nan_step, sizeof(int))) || (rc = c->dalloc((void **)&c->acq.l2, sizeof(double) * l2_scratch_doubles())))
+    if ((rc = c->dalloc((void **)&c->acq.nan_step, 2 * sizeof(int))) || (rc = c->dalloc((void **)&c->acq.l2, sizeof(double) * l2_scratch_doubles())))
         return bail(rc);
     c->acq.nt = p->nt;
     c->tile_v = c->tile_s = default_tile(p->nx, p->ny);
+    c->res_pool = res_pool_open(device);
+    if (c->res_pool) c->res = res_plan(*p, res_pool_cus(c->res_pool), res_pool_lds(c->res_pool));
     if ((rc = build_lists(c))) return bail(rc);
     fill_args(c);
     if (hipStreamSynchronize(c->stream) != hipSuccess) return bail(fail(DN_ERR_HIP, "stream synchronisation failed"));
@@ -914,6 +1058,7 @@ int dn_set_tile(dn_ctx *c, int sweep, int tbx, int by, int ty, int vw)
     HIP_OK(hipStreamSynchronize(c->stream));
     if (sweep != 1) c->tile_v = t;
     if (sweep != 0) c->tile_s = t;
+    c->sweeps_chosen = true;
     return build_lists(c);
 }
 
@@ -935,6 +1080,7 @@ int dn_autotune_tile(dn_ctx *c, int nsteps, int *vel_shape, int *str_shape)
     Tile shapes[32];
     const int n = tile_list(shapes, 32);
     const int keep_sampling = c->sample_every;
+    const bool keep_chosen = c->sweeps_chosen;  // the tuned shapes serve the runs that take the sweeps
     c->sample_every = 1;  // time every launch of both sweeps
     Tile best_v = c->tile_v, best_s = c->tile_s;
     double bv = -1.0, bs = -1.0;
@@ -986,6 +1132,7 @@ int dn_autotune_tile(dn_ctx *c, int nsteps, int *vel_shape, int *str_shape)
         c->nt_s = hs;
     }
     c->sample_every = keep_sampling;
+    c->sweeps_chosen = keep_chosen;
     if (rc) return rc;
     c->tile_v = best_v;
     c->tile_s = best_s;
@@ -1010,6 +1157,7 @@ int dn_set_store_hint(dn_ctx *c, int sweep, int streaming)
         return fail(DN_ERR_ARG, "bad store hint");
     if (sweep != 1) c->nt_v = streaming;
     if (sweep != 0) c->nt_s = streaming;
+    c->sweeps_chosen = true;
     return DN_OK;
 }
 
@@ -1090,6 +1238,16 @@ int dn_run_forward(dn_ctx *c, int nsteps)
     if (c->eprecond)  // grad_obj_psv.c:71-76: the energies start at zero for each shot
         for (int w = 0; w < 2; ++w) HIP_OK(hipMemsetAsync(c->ew[w], 0, (size_t)c->p.nx * c->p.ny * sizeof(float), c->stream));
     HIP_OK(hipEventRecord(c->ev0, c->stream));
+    if (res_applies(c, 0)) {
+        bool done = false;
+        if ((rc = res_run(c, ctl, 0, nsteps, &done))) return rc;
+        if (done) {
+            c->fwd_complete = fwdstore && nsteps == NT;
+            return DN_OK;
+        }
+        if ((rc = zero_state(c))) return rc;
+        HIP_OK(hipEventRecord(c->ev0, c->stream));
+    }
     int hin = 1, hin1 = 1, lsnap = c->snap_first, nsnap = 0;
     std::vector<float> snapbuf;
     for (int nt = 1; nt <= nsteps; ++nt) {
@@ -1227,14 +1385,22 @@ int dn_run_adjoint(dn_ctx *c, int nsteps)
     int rc = zero_state(c);
     if (rc) return rc;
     const size_t g = (size_t)c->p.nx * c->p.ny * sizeof(float);
-    HIP_OK(hipMemsetAsync(c->wc, 0, g, c->stream));
-    HIP_OK(hipMemsetAsync(c->wcu, 0, g, c->stream));
-    HIP_OK(hipMemsetAsync(c->wcr, 0, g, c->stream));
+    auto zero_sums = [&]() -> int {
+        for (float *w : {c->wc, c->wcu, c->wcr}) HIP_OK(hipMemsetAsync(w, 0, g, c->stream));
+        return DN_OK;
+    };
+    if ((rc = zero_sums())) return rc;
     KArgs av = c->a, as = c->a;
     StepCtl ctl = base_ctl(c, 2, 3);
     ctl.probe = 1;
     size_t nev = 0;
     HIP_OK(hipEventRecord(c->ev0, c->stream));
+    if (res_applies(c, 1)) {
+        bool done = false;
+        if ((rc = res_run(c, ctl, 1, nsteps, &done)) || done) return rc;
+        if ((rc = zero_state(c)) || (rc = zero_sums())) return rc;
+        HIP_OK(hipEventRecord(c->ev0, c->stream));
+    }
     int hin = 1;
     for (int nt = 1; nt <= nsteps; ++nt) {
         const bool sample = c->sample_every > 0 && (nt % c->sample_every) == 0;

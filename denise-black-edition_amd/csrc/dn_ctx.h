@@ -9,6 +9,7 @@
 
 #include "dn_arena.h"
 #include "dn_internal.h"
+#include "dn_resident.h"
 
 namespace dn {
 // records the message for dn_last_error() and returns code
@@ -82,6 +83,16 @@ struct dn_ctx {
     Ent *lst_ent[4] = {};
     int lst_nlean[4] = {}, lst_nfull[4] = {};
     std::vector<int> lean_h[4], full_h[4];  // host copies of the tile sets
+    // chip-resident runs: the grid's cut, its sources and receivers per tile
+    // (lists as above), and whether the caller asked for the sweeps by
+    // choosing their shape or cache policy
+    ResPool *res_pool = nullptr;
+    ResPlan res;
+    bool sweeps_chosen = false;
+    int *res_lst = nullptr;  // one block: per list offsets, owners, entries
+    size_t res_off[4] = {}, res_own[4] = {}, res_ent[4] = {};  // positions in it (ints)
+    bool res_lst_ok[4] = {};
+    int res_most[4] = {};  // entries of a tile, at most
     // timing
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double run_ms = 0.0, v_ms = 0.0, s_ms = 0.0;
@@ -146,6 +157,7 @@ struct dn_ctx {
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         if (stream) (void)hipStreamDestroy(stream);
+        res_pool_close(res_pool);
     }
 };
 

@@ -1,0 +1,60 @@
+// Chip-resident time loop (dn_resident.inc): launch arguments and the pool of
+// halo mailboxes.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "dn_resident_plan.h"
+
+namespace dn {
+
+typedef unsigned long long res_word;
+
+struct ResArgs {
+    int tw, th, gx, gy, nthx, ncomp, nk_s, nk_v, cap, ncx, ncy, nve, nse;
+    int n0, n1, nlast;  // time steps of this launch, last step of the run
+    int fwdstore, dtinv, vp1_form;
+    bool vec;           // snapshot rows keep 16-byte alignment
+    double rdh;         // 1 / DH
+    unsigned tag0;
+    res_word *mbox;
+    int *abort;
+    // sources and receivers per tile, sorted by owner thread:
+    // {kind << 24 | LDS element, index}
+    const int *voff, *vown, *soff, *sown;
+    const uint2 *vent, *sent;
+};
+
+// the kernel's one argument
+struct ResKernel {
+    KArgs a;
+    StepCtl c;
+    DevAcq q;
+    ResArgs r;
+};
+
+// is there a compiled kernel for this run (sw 0 forward, 1 adjoint)
+bool res_compiled(int physics, int L, int sw);
+// enqueue one launch; false when the runtime refuses it
+bool res_launch(const KArgs &a, const StepCtl &c, const DevAcq &q, const ResArgs &r, const ResPlan &pl, int fdoh,
+                int sw, void *stream);
+
+// The mailboxes of a device: one allocation shared by the contexts on it,
+// made with the first and given back with the last, and the account of its
+// CUs.  A run takes a range of mailboxes and as many CUs as it has tiles for
+// its duration; runs that find too few take the sweeps instead of waiting,
+// so runs of several threads and streams never wait for each other's CUs.
+// Step tags only grow, so a word left by an earlier run matches no later
+// tag.  Thread-safe.
+struct ResPool;
+ResPool *res_pool_open(int device);  // nullptr: no pool (no memory)
+void res_pool_close(ResPool *p);
+int res_pool_cus(const ResPool *p);
+size_t res_pool_lds(const ResPool *p);
+struct ResLease {
+    res_word *mbox = nullptr;
+    unsigned tag0 = 0;
+};
+bool res_pool_take(ResPool *p, const ResPlan &pl, int steps, ResLease *out);
+void res_pool_give(ResPool *p, const ResLease &l);
+
+}  // namespace dn

@@ -1,0 +1,139 @@
+"""The chip-resident time loop (dn_resident.*) against the sweeps and the FP32
+oracle: one grid per thread shape (1x1, 1x2, 1x4, 2x4, 3x4 cells per thread)
+with ragged last tiles, every operator length, points on tile edges, runs
+longer than one launch.  A context whose caller chose a sweep shape takes the
+sweeps; all other runs here fit the loop.  The arithmetic is the same term by
+term, so everything compares bit for bit."""
+import numpy as np
+import pytest
+
+import dnhip
+import orc
+from cases import make_case
+
+pytestmark = pytest.mark.gpu
+
+
+def context(case, sweeps):
+    p, m, src, sig, rec = case
+    g = dnhip.Context(p)
+    g.set_model(m["vp"], m["vs"], m["rho"], m["taus"], m["taup"])
+    if sweeps:
+        g.set_tile(64, 4, 1, 1)
+    g.set_sources(src, sig)
+    g.set_receivers(rec)
+    return g
+
+
+def state(g, p):
+    out = [g.seismogram(k) for k in range(5)] + [g.field(f) for f in range(7)] + [g.psi(k) for k in range(9)]
+    return out + [g.memvar(w, l + 1) for w in range(3) for l in range(p.L)]
+
+
+def check_forward(case, steps=0):
+    a, b = context(case, False), context(case, True)
+    print(f"resident run {case[0].nx}x{case[0].ny} order {case[0].fdorder}", flush=True)
+    a.forward(steps)
+    b.forward(steps)
+    assert np.abs(a.field(dnhip.F_VX)).max() > 0
+    for k, (x, y) in enumerate(zip(state(a, case[0]), state(b, case[0]))):
+        np.testing.assert_array_equal(x, y, err_msg=f"output {k}")
+    return a
+
+
+# grids: one tile; ragged tiles of 1x1, 1x2, 1x4, 2x4 and 3x4 cells per thread
+GRIDS = [(29, 21), (131, 77), (611, 303), (1003, 401), (1201, 601), (1502, 602), (1997, 598)]
+
+
+@pytest.mark.parametrize("free_surf", [0, 1])
+@pytest.mark.parametrize("nx,ny", GRIDS)
+def test_forward_equals_sweeps_on_every_thread_shape(nx, ny, free_surf):
+    fw = 5 if ny < 40 else 10
+    check_forward(make_case(nx=nx, ny=ny, nt=60, fdorder=8, fw=fw, free_surf=free_surf, seismo=4, homogeneous=True,
+                            nrec=max(3, nx // 2 - 4)))
+
+
+@pytest.mark.parametrize("fdorder", [2, 4, 6, 8, 10, 12])
+def test_forward_equals_oracle_for_every_order(fdorder):
+    case = make_case(nx=173, ny=61, nt=150, fdorder=fdorder, fw=7, seismo=4, free_surf=fdorder // 2 % 2)
+    g = check_forward(case)
+    p, m, src, sig, rec = case
+    o = orc.Oracle(p, m["vp"], m["vs"], m["rho"], prec="f32")
+    o.set_sources(src, sig)
+    o.set_receivers(rec)
+    o.forward()
+    for k in range(5):
+        np.testing.assert_array_equal(g.seismogram(k), o.seismogram(k))
+
+
+@pytest.mark.parametrize("stype", [1, 2, 3, 4])
+def test_points_on_tile_edges(stype):
+    """Sources and receivers in the last and first cells of tiles (32 columns
+    and up to 32 rows), the grid's corners among them, several per cell."""
+    case = make_case(nx=140, ny=90, nt=120, fw=10, seismo=4, stype=stype)
+    p, m, src, sig, rec = case
+    src = np.repeat(src, 3, 1)
+    src[0] = [32, 33, 33]
+    src[1] = [2, 40, 40]
+    sig = np.repeat(sig, 3, 0) * np.array([[1.0], [0.5], [-0.25]], np.float32)
+    xs = [1, 31, 32, 33, 64, 65, 96, 97, 139, 140]
+    ys = [1, 2, 3, 4, 5, 6, 9, 44, 89, 90]
+    rec = np.array([[x for x in xs for _ in ys], [y for _ in xs for y in ys]], np.int32)
+    check_forward((p, m, src, sig, rec))
+
+
+def test_surface_source_and_long_runs():
+    """An explosive source in the surface row (applied before the surface
+    condition: the sweeps take it), and a run of several launches."""
+    case = make_case(nx=90, ny=60, nt=100, src_xz=(450.0, 10.0))
+    check_forward(case)
+    check_forward(make_case(nx=90, ny=60, nt=4500, fw=10))
+    check_forward(make_case(nx=90, ny=60, nt=400, fw=10), steps=33)
+
+
+@pytest.mark.parametrize("nx,ny,dtinv", [(131, 77, 1), (256, 120, 3), (612, 302, 2), (1201, 601, 4)])
+def test_stored_snapshots_give_the_sweeps_gradient(nx, ny, dtinv):
+    case = make_case(nx=nx, ny=ny, nt=90, fw=10, mode=1, dtinv=dtinv, homogeneous=True)
+    grads = []
+    for sweeps in (False, True):
+        g = context(case, sweeps)
+        print(f"resident snapshots {nx}x{ny} dtinv {dtinv} sweeps {sweeps}", flush=True)
+        g.forward()
+        z = np.zeros((g.ntr, case[0].nt), np.float32)
+        l2 = g.residuals(z, z)
+        g.adjoint()
+        g.assemble()
+        grads.append([np.float64(l2)] + [g.gradient(k) for k in range(6)] +
+                     [g.field(f) for f in range(7)] + [g.psi(k) for k in range(9)])
+        g.close()
+    assert np.abs(grads[0][4]).max() > 0
+    for x, y in zip(*grads):
+        np.testing.assert_array_equal(x, y)
+
+
+def test_concurrent_contexts():
+    """More runs at once than the CUs take: those without room take the
+    sweeps, and every result is the run's own."""
+    import threading
+    cases = [make_case(nx=400 + 20 * k, ny=200, nt=150, fw=10, seed=k + 1) for k in range(4)]
+    want = []
+    for c in cases:
+        g = context(c, True)
+        g.forward()
+        want.append(g.seismogram(0))
+    ctx = [context(c, False) for c in cases]
+    bad = []
+
+    def work(k):
+        for _ in range(3):
+            ctx[k].forward()
+            if not np.array_equal(ctx[k].seismogram(0), want[k]):
+                bad.append(k)
+
+    print("concurrent resident runs", flush=True)
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
