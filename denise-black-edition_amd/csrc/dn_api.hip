@@ -507,7 +507,6 @@ int res_run(dn_ctx *c, const StepCtl &ctl, int sw, int nsteps, bool *done)
     r.fwdstore = c->p.mode > 0;
     r.dtinv = c->p.dtinv > 0 ? c->p.dtinv : 1;
     r.vp1_form = c->p.grad_form == 1 || c->p.grad_form == 2;
-    r.vec = c->p.nx % 4 == 0;
     r.rdh = 1.0 / (double)c->p.dh;
     r.mbox = l.mbox;
     r.abort = c->acq.nan_step + 1;

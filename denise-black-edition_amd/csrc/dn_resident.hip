@@ -28,7 +28,7 @@ bool res_launch(const KArgs &a, const StepCtl &c, const DevAcq &q, const ResArgs
     return false;
 }
 
-bool res_compiled(int physics, int L, int sw) { return physics == 1 && L == 0 && sw == 0; }
+bool res_compiled(int physics, int L, int sw) { (void)sw; return physics == 1 && L == 0; }
 
 // ---------------------------------------------------------------- the pool
 struct ResPool {
