@@ -470,6 +470,9 @@ bool res_applies(const dn_ctx *c, int sw)
     if (!c->res_lst_ok[2 * sw] || !c->res_lst_ok[2 * sw + 1]) return false;
     if (c->res_most[2 * sw] > RES_ENT || c->res_most[2 * sw + 1] > RES_ENT) return false;
     if (res_lds(c, sw) > res_pool_lds(c->res_pool)) return false;
+    // the curl at acoustic receivers differences vx along y and vy along x,
+    // halo cells that the acoustic update does not need
+    if (c->a.physics == 2 && c->p.seismo >= 3) return false;
     if (c->qtype == 5 || c->eprecond || c->snap_fn || c->sample_every > 0) return false;
     if (c->p.mode > 0 && c->p.grad_form != 1) return false;
     for (int k : {P_KX, P_KXH, P_KY, P_KYH})

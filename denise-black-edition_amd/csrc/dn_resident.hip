@@ -9,7 +9,7 @@
 
 namespace dn {
 
-template <int F>
+template <int F, int GROUP>
 bool res_launch_f(const KArgs &a, const StepCtl &c, const DevAcq &q, const ResArgs &r, const ResPlan &pl, int sw,
                   hipStream_t s);
 
@@ -17,18 +17,22 @@ bool res_launch(const KArgs &a, const StepCtl &c, const DevAcq &q, const ResArgs
                 int sw, void *stream)
 {
     hipStream_t s = (hipStream_t)stream;
+#define DN_F(F)                                                      \
+    case F:                                                          \
+        return a.physics == 1 ? res_launch_f<F, 0>(a, c, q, r, pl, sw, s) \
+                              : res_launch_f<F, 1>(a, c, q, r, pl, sw, s);
     switch (fdoh) {
-    case 1: return res_launch_f<1>(a, c, q, r, pl, sw, s);
-    case 2: return res_launch_f<2>(a, c, q, r, pl, sw, s);
-    case 3: return res_launch_f<3>(a, c, q, r, pl, sw, s);
-    case 4: return res_launch_f<4>(a, c, q, r, pl, sw, s);
-    case 5: return res_launch_f<5>(a, c, q, r, pl, sw, s);
-    case 6: return res_launch_f<6>(a, c, q, r, pl, sw, s);
+        DN_F(1) DN_F(2) DN_F(3) DN_F(4) DN_F(5) DN_F(6)
     }
+#undef DN_F
     return false;
 }
 
-bool res_compiled(int physics, int L, int sw) { (void)sw; return physics == 1 && L == 0; }
+bool res_compiled(int physics, int L, int sw)
+{
+    (void)sw;
+    return physics >= 1 && physics <= 5 && L == 0;
+}
 
 // ---------------------------------------------------------------- the pool
 struct ResPool {

@@ -28,7 +28,7 @@ ResPlan res_plan(const dn_params &p, int ncu, size_t lds_max)
     for (const auto &sh : shapes) {
         if (best.ok) break;
         double cost = 0.0;
-        const int ry = sh[0], maxt = res_maxt(sh[0], sh[1], F);
+        const int ry = sh[0], maxt = res_maxt(sh[0], sh[1], F, p.L);
         ResPlan q;
         q.ry = ry;
         q.vx = sh[1];

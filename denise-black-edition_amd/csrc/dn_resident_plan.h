@@ -18,9 +18,9 @@ namespace dn {
 // 32 columns wide, 2 x 4 or 3 x 4 in tiles up to 64 or 72 wide; the
 // widest tile fixes the LDS pitch at compile time.  A workgroup has as many threads as
 // the registers of that shape allow without spilling.
-constexpr int res_maxt(int ry, int vx, int F)
+constexpr int res_maxt(int ry, int vx, int F, int L)
 {
-    return ry > 1 ? 512 : vx == 1 ? 1024 : vx == 2 ? (F <= 4 ? 1024 : 768) : (F <= 4 ? 768 : 512);
+    return ry > 1 ? 512 : vx == 1 ? 1024 : vx == 2 ? (F <= 4 ? 1024 : 768) : (F <= 4 && L == 0 ? 768 : 512);
 }
 constexpr int res_width(int ry) { return ry == 1 ? 32 : ry == 2 ? 64 : 72; }
 constexpr int RES_ENT = 256;     // sources and receivers of one tile and sweep kept in LDS, at most

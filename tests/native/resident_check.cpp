@@ -24,7 +24,7 @@ static void check(const dn_params &p, const ResPlan &pl)
     constexpr int HP = 4 * ((F + 3) / 4), LP = TW + 2 * HP;
     const int nf = res_planes(PH);
     const ResCut cut{pl.gx, pl.gy, pl.tw, pl.th, pl.cap};
-    CHECK(pl.tw <= TW && pl.tw % 4 == 0 && pl.tw >= 8 && pl.nthr <= res_maxt(pl.ry, pl.vx, F) && pl.nthr % 64 == 0 && pl.ncomp <= pl.nthr && pl.tiles() <= 256);
+    CHECK(pl.tw <= TW && pl.tw % 4 == 0 && pl.tw >= 8 && pl.nthr <= res_maxt(pl.ry, pl.vx, F, p.L) && pl.nthr % 64 == 0 && pl.ncomp <= pl.nthr && pl.tiles() <= 256);
     CHECK((pl.gx - 1) * pl.tw < p.nx && pl.gx * pl.tw >= p.nx && (pl.gy - 1) * pl.th < p.ny && pl.gy * pl.th >= p.ny);
     CHECK(pl.th % pl.ry == 0 && pl.nthx * pl.vx == pl.tw && pl.ncomp == pl.nthx * (pl.th / pl.ry));
     CHECK(pl.cap <= RES_CAP && pl.lds <= 163840);

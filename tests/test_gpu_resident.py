@@ -9,6 +9,7 @@ import pytest
 
 import dnhip
 import orc
+import synth
 from cases import make_case
 
 pytestmark = pytest.mark.gpu
@@ -17,7 +18,11 @@ pytestmark = pytest.mark.gpu
 def context(case, sweeps):
     p, m, src, sig, rec = case
     g = dnhip.Context(p)
-    g.set_model(m["vp"], m["vs"], m["rho"], m["taus"], m["taup"])
+    if p.physics in (3, 4):
+        g.set_model_aniso(*synth.anisotropic_model(p.nx, p.ny, p.dh, 5, sigma=3.0,
+                                                   tilt=20.0 if p.physics == 4 else None))
+    else:
+        g.set_model(m["vp"], m["vs"], m["rho"], m["taus"], m["taup"])
     if sweeps:
         g.set_tile(64, 4, 1, 1)
     g.set_sources(src, sig)
@@ -91,24 +96,53 @@ def test_surface_source_and_long_runs():
     check_forward(make_case(nx=90, ny=60, nt=400, fw=10), steps=33)
 
 
-@pytest.mark.parametrize("nx,ny,dtinv", [(131, 77, 1), (256, 120, 3), (612, 302, 2), (1201, 601, 4)])
-def test_stored_snapshots_give_the_sweeps_gradient(nx, ny, dtinv):
-    case = make_case(nx=nx, ny=ny, nt=90, fw=10, mode=1, dtinv=dtinv, homogeneous=True)
-    grads = []
-    for sweeps in (False, True):
-        g = context(case, sweeps)
-        print(f"resident snapshots {nx}x{ny} dtinv {dtinv} sweeps {sweeps}", flush=True)
-        g.forward()
-        z = np.zeros((g.ntr, case[0].nt), np.float32)
-        l2 = g.residuals(z, z)
-        g.adjoint()
+def gradient(case, sweeps):
+    g = context(case, sweeps)
+    print(f"resident gradient physics {case[0].physics} {case[0].nx}x{case[0].ny} sweeps {sweeps}", flush=True)
+    g.forward()
+    seis = [g.seismogram(k) for k in range(5)]
+    rng = np.random.default_rng(3)
+    adj = [(rng.standard_normal((g.ntr, case[0].nt)) * 1e-6).astype(np.float32) for _ in range(3)]
+    g.set_adjoint_sources(*adj)
+    g.adjoint()
+    out = seis + [g.gradient(k) for k in range(3)] + [g.field(f) for f in range(7)] + [g.psi(k) for k in range(9)]
+    if case[0].physics not in (3, 4):
         g.assemble()
-        grads.append([np.float64(l2)] + [g.gradient(k) for k in range(6)] +
-                     [g.field(f) for f in range(7)] + [g.psi(k) for k in range(9)])
-        g.close()
-    assert np.abs(grads[0][4]).max() > 0
-    for x, y in zip(*grads):
+        out += [g.gradient(k) for k in range(3, 6)]
+    g.close()
+    return out
+
+
+@pytest.mark.parametrize("nx,ny,dtinv", [(131, 77, 1), (256, 120, 3), (612, 302, 2), (1201, 601, 4), (1997, 598, 3)])
+def test_gradient_equals_sweeps(nx, ny, dtinv):
+    """Stored snapshots and the adjoint run with its correlations, odd NX and
+    the unaligned snapshot rows it brings among them."""
+    case = make_case(nx=nx, ny=ny, nt=70, fw=10, mode=1, dtinv=dtinv, homogeneous=True)
+    a, b = gradient(case, False), gradient(case, True)
+    assert np.abs(a[5]).max() > 0
+    for x, y in zip(a, b):
         np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("quelltypb", [1, 2, 3, 4, 7])
+def test_adjoint_source_types(quelltypb):
+    case = make_case(nx=140, ny=90, nt=80, fw=10, mode=1, dtinv=2, quelltypb=quelltypb, seismo=4)
+    for x, y in zip(gradient(case, False), gradient(case, True)):
+        np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("nx,ny,fdorder,free_surf", [(29, 21, 4, 1), (140, 90, 2, 0), (173, 61, 12, 1),
+                                                     (811, 303, 8, 1), (1201, 601, 8, 0), (1997, 598, 8, 1)])
+@pytest.mark.parametrize("physics", [2, 3, 4, 5])
+def test_other_physics_equal_sweeps(physics, nx, ny, fdorder, free_surf):
+    """Acoustic, VTI, TTI and SH runs, forward with snapshots and adjoint."""
+    case = make_case(nx=nx, ny=ny, nt=60, fdorder=fdorder, fw=5 if ny < 40 else 10, mode=1, dtinv=2, safety=0.5,
+                     free_surf=free_surf, seismo={2: 2, 5: 1}.get(physics, 4), homogeneous=True)
+    case[0].physics = physics
+    a, b = gradient(case, False), gradient(case, True)
+    assert max(np.abs(x).max() for x in a[5:8]) > 0
+    for k, (x, y) in enumerate(zip(a, b)):
+        np.testing.assert_array_equal(x, y, err_msg=f"output {k}")
 
 
 def test_concurrent_contexts():
