@@ -254,13 +254,9 @@ int build_lists(dn_ctx *c)
             off.insert(off.end(), slot.begin(), slot.end());
             off.insert(off.end(), lo.begin(), lo.end());
         }
-        if (c->lst_off[w]) c->dfree(c->lst_off[w]);
-        if (c->lst_ent[w]) c->dfree(c->lst_ent[w]);
-        c->lst_off[w] = nullptr;
-        c->lst_ent[w] = nullptr;
         int rc;
-        if ((rc = c->dalloc((void **)&c->lst_off[w], off.size() * sizeof(int))) ||
-            (rc = c->dalloc((void **)&c->lst_ent[w], ent.size() * sizeof(Ent))))
+        if ((rc = c->regrow((void **)&c->lst_off[w], off.size() * sizeof(int))) ||
+            (rc = c->regrow((void **)&c->lst_ent[w], ent.size() * sizeof(Ent))))
             return rc;
         HIP_OK(h2d(c->stream, c->lst_off[w], off.data(), off.size() * sizeof(int)));
         HIP_OK(h2d(c->stream, c->lst_ent[w], ent.data(), ent.size() * sizeof(Ent)));
@@ -305,10 +301,8 @@ int build_lists(dn_ctx *c)
             blk.push_back(o.idx);
         }
     }
-    if (c->res_lst) c->dfree(c->res_lst);
-    c->res_lst = nullptr;
     int rc;
-    if ((rc = c->dalloc((void **)&c->res_lst, blk.size() * sizeof(int)))) return rc;
+    if ((rc = c->regrow((void **)&c->res_lst, blk.size() * sizeof(int)))) return rc;
     HIP_OK(h2d(c->stream, c->res_lst, blk.data(), blk.size() * sizeof(int)));
     return DN_OK;
 }
@@ -470,6 +464,7 @@ bool res_applies(const dn_ctx *c, int sw)
     if (!c->res_lst_ok[2 * sw] || !c->res_lst_ok[2 * sw + 1]) return false;
     if (c->res_most[2 * sw] > RES_ENT || c->res_most[2 * sw + 1] > RES_ENT) return false;
     if (res_lds(c, sw) > res_pool_lds(c->res_pool)) return false;
+    if (c->p.L > 0 && !c->tau_const) return false;  // relaxation times as planes
     // the curl at acoustic receivers differences vx along y and vy along x,
     // halo cells that the acoustic update does not need
     if (c->a.physics == 2 && c->p.seismo >= 3) return false;

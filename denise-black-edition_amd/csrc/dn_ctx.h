@@ -148,6 +148,16 @@ struct dn_ctx {
                 return;
             }
     }
+    // a buffer of at least nbytes: the one there if it is large enough (the
+    // cell lists are rebuilt for every shot), else a new one
+    int regrow(void **ptr, size_t nbytes)
+    {
+        for (auto &pr : allocs)
+            if (*ptr && pr.first == *ptr && pr.second >= nbytes) return DN_OK;
+        if (*ptr) dfree(*ptr);
+        *ptr = nullptr;
+        return dalloc(ptr, nbytes);
+    }
     ~dn_ctx()
     {
         if (device >= 0) (void)hipSetDevice(device);

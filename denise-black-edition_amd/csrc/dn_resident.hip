@@ -19,8 +19,9 @@ bool res_launch(const KArgs &a, const StepCtl &c, const DevAcq &q, const ResArgs
     hipStream_t s = (hipStream_t)stream;
 #define DN_F(F)                                                      \
     case F:                                                          \
-        return a.physics == 1 ? res_launch_f<F, 0>(a, c, q, r, pl, sw, s) \
-                              : res_launch_f<F, 1>(a, c, q, r, pl, sw, s);
+        return a.physics != 1 ? res_launch_f<F, 1>(a, c, q, r, pl, sw, s) \
+               : a.L > 0      ? res_launch_f<F, 2>(a, c, q, r, pl, sw, s) \
+                              : res_launch_f<F, 0>(a, c, q, r, pl, sw, s);
     switch (fdoh) {
         DN_F(1) DN_F(2) DN_F(3) DN_F(4) DN_F(5) DN_F(6)
     }
@@ -31,7 +32,7 @@ bool res_launch(const KArgs &a, const StepCtl &c, const DevAcq &q, const ResArgs
 bool res_compiled(int physics, int L, int sw)
 {
     (void)sw;
-    return physics >= 1 && physics <= 5 && L == 0;
+    return physics >= 1 && physics <= 5 && (L == 0 || (physics == 1 && L <= 3));
 }
 
 // ---------------------------------------------------------------- the pool

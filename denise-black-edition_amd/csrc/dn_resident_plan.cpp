@@ -26,7 +26,7 @@ ResPlan res_plan(const dn_params &p, int ncu, size_t lds_max)
     // 2 x 4; 611x303 5.9 with 1 x 2, 7.6 with 1 x 4, 10.2 with 2 x 4.
     static const int shapes[][2] = {{1, 1}, {1, 2}, {1, 4}, {2, 4}, {3, 4}};
     for (const auto &sh : shapes) {
-        if (best.ok) break;
+        if (best.ok || sh[0] > res_rows(p.L)) break;
         double cost = 0.0;
         const int ry = sh[0], maxt = res_maxt(sh[0], sh[1], F, p.L);
         ResPlan q;

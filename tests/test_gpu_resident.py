@@ -145,6 +145,18 @@ def test_other_physics_equal_sweeps(physics, nx, ny, fdorder, free_surf):
         np.testing.assert_array_equal(x, y, err_msg=f"output {k}")
 
 
+@pytest.mark.parametrize("L", [1, 2, 3])
+@pytest.mark.parametrize("nx,ny,fdorder,free_surf", [(140, 90, 8, 1), (331, 303, 12, 0), (1003, 401, 8, 1),
+                                                     (1201, 601, 4, 1), (1997, 598, 8, 1)])
+def test_viscoelastic_equals_sweeps(L, nx, ny, fdorder, free_surf):
+    """Forward runs with their memory variables, and gradients."""
+    kw = dict(nx=nx, ny=ny, nt=60, fdorder=fdorder, fw=10, L=L, free_surf=free_surf, seismo=4, homogeneous=True)
+    check_forward(make_case(**kw))
+    case = make_case(mode=1, dtinv=2, **kw)
+    for k, (x, y) in enumerate(zip(gradient(case, False), gradient(case, True))):
+        np.testing.assert_array_equal(x, y, err_msg=f"output {k}")
+
+
 def test_concurrent_contexts():
     """More runs at once than the CUs take: those without room take the
     sweeps, and every result is the run's own."""
