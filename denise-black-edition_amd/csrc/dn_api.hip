@@ -148,40 +148,15 @@ Tile default_tile(int nx, int ny)
     return t;
 }
 
-// Per-tile cell work lists of the two sweeps (see Ent in dn_internal.h).
-int build_lists(dn_ctx *c)
+// a source or receiver cell of list `which` (see dn_ctx.h)
+struct Point {
+    int which, i, j, kind, idx;
+};
+
+std::vector<Point> points(const dn_ctx *c)
 {
-    const int NX = c->p.nx, NY = c->p.ny;
-    c->ntx_v = c->tile_v.ntx(NX);
-    c->ntiles_v = c->ntx_v * c->tile_v.nty(NY);
-    c->ntx_s = c->tile_s.ntx(NX);
-    c->ntiles_s = c->ntx_s * c->tile_s.nty(NY);
-    struct Item {
-        int tile;
-        Ent e;
-    };
-    std::vector<Item> lists[4];
-    // lists 0 and 2 belong to the velocity sweep, 1 and 3 to the stress sweep
-    auto add_tile = [&](int which, int i, int j, int kind, int idx) {
-        const Tile &t = (which == 0 || which == 2) ? c->tile_v : c->tile_s;
-        const int ntx = (which == 0 || which == 2) ? c->ntx_v : c->ntx_s;
-        const int tx = (i - 1) / t.width(), ty = (j - 1) / t.rows();
-        Item it;
-        it.tile = ty * ntx + tx;
-        it.e.lane = (i - 1) - tx * t.width();
-        it.e.row = j;
-        it.e.kind = kind;
-        it.e.idx = idx;
-        lists[which].push_back(it);
-    };
-    struct Point {
-        int which, i, j, kind, idx;
-    };
-    std::vector<Point> points;
-    auto add = [&](int which, int i, int j, int kind, int idx) {
-        add_tile(which, i, j, kind, idx);
-        if (c->res.ok) points.push_back(Point{which, i, j, kind, idx});
-    };
+    std::vector<Point> v;
+    auto add = [&](int which, int i, int j, int kind, int idx) { v.push_back(Point{which, i, j, kind, idx}); };
     const int ns = (int)c->src_ix.size(), nr = (int)c->rec_ix.size();
     const int seismo = c->p.seismo;
     // SH: QUELLTYP 1 is the force on vz (update_v_PML_SH.c:560-568); the SH
@@ -199,6 +174,35 @@ int build_lists(dn_ctx *c)
     for (int r = 0; r < nr; ++r) add(2, c->rec_ix[r], c->rec_iy[r], E_ADJ_FORCE, r);
     if (c->p.quelltypb >= 4)
         for (int r = 0; r < nr; ++r) add(3, c->rec_ix[r], c->rec_iy[r], E_ADJ_P, r);
+    return v;
+}
+
+// Per-tile cell work lists of the two sweeps (see Ent in dn_internal.h).
+int build_lists(dn_ctx *c)
+{
+    const int NX = c->p.nx, NY = c->p.ny;
+    c->ntx_v = c->tile_v.ntx(NX);
+    c->ntiles_v = c->ntx_v * c->tile_v.nty(NY);
+    c->ntx_s = c->tile_s.ntx(NX);
+    c->ntiles_s = c->ntx_s * c->tile_s.nty(NY);
+    struct Item {
+        int tile;
+        Ent e;
+    };
+    std::vector<Item> lists[4];
+    // lists 0 and 2 belong to the velocity sweep, 1 and 3 to the stress sweep
+    for (const Point &q : points(c)) {
+        const Tile &t = (q.which == 0 || q.which == 2) ? c->tile_v : c->tile_s;
+        const int ntx = (q.which == 0 || q.which == 2) ? c->ntx_v : c->ntx_s;
+        const int tx = (q.i - 1) / t.width(), ty = (q.j - 1) / t.rows();
+        Item it;
+        it.tile = ty * ntx + tx;
+        it.e.lane = (q.i - 1) - tx * t.width();
+        it.e.row = q.j;
+        it.e.kind = q.kind;
+        it.e.idx = q.idx;
+        lists[q.which].push_back(it);
+    }
     for (int w = 0; w < 4; ++w) {
         // by tile, then lane; entries of one cell keep their order
         std::stable_sort(lists[w].begin(), lists[w].end(), [](const Item &x, const Item &y) {
@@ -262,20 +266,32 @@ int build_lists(dn_ctx *c)
         HIP_OK(h2d(c->stream, c->lst_ent[w], ent.data(), ent.size() * sizeof(Ent)));
     }
     if (!c->res.ok) return DN_OK;
-    // the same points by tile and owner thread of the chip-resident loop
-    const ResPlan &pl = c->res;
+    res_points(c, c->res, &c->res_pts);
+    int rc;
+    if ((rc = c->regrow((void **)&c->res_lst, c->res_pts.blk.size() * sizeof(int)))) return rc;
+    HIP_OK(h2d(c->stream, c->res_lst, c->res_pts.blk.data(), c->res_pts.blk.size() * sizeof(int)));
+    return DN_OK;
+}
+
+}  // namespace
+
+// the sources and receivers by tile and owner thread of a plan
+void dn::res_points(const dn_ctx *c, const ResPlan &pl, ResPoints *o)
+{
     const int HP = 4 * ((c->fdoh + 3) / 4), LP = res_width(pl.ry) + 2 * HP;
-    std::vector<int> blk;
+    const std::vector<Point> all = points(c);
+    std::vector<int> &blk = o->blk;
+    blk.clear();
     for (int w = 0; w < 4; ++w) {
         struct Own {
             int tile, own, el, kind, idx;
         };
         std::vector<Own> v;
-        c->res_lst_ok[w] = true;
-        for (const Point &q : points) {
+        o->ok[w] = true;
+        for (const Point &q : all) {
             if (q.which != w) continue;
             // the surface condition of row 1 follows the sources added there
-            if (q.j == 1 && c->a.mirror && (q.kind == E_EXPLOSIVE || q.kind == E_ADJ_P)) c->res_lst_ok[w] = false;
+            if (q.j == 1 && c->a.mirror && (q.kind == E_EXPLOSIVE || q.kind == E_ADJ_P)) o->ok[w] = false;
             const int bx = (q.i - 1) / pl.tw, by = (q.j - 1) / pl.th;
             const int x = q.i - 1 - bx * pl.tw, y = q.j - 1 - by * pl.th;
             v.push_back(Own{by * pl.gx + bx, y / pl.ry * pl.nthx + x / pl.vx, (y + c->fdoh) * LP + HP + x, q.kind, q.idx});
@@ -284,30 +300,24 @@ int build_lists(dn_ctx *c)
             return x.tile < y.tile || (x.tile == y.tile && x.own < y.own);
         });
         std::vector<int> off((size_t)pl.tiles() + 1, 0);
-        for (const Own &o : v) off[(size_t)o.tile + 1]++;
-        c->res_most[w] = 0;
+        for (const Own &p : v) off[(size_t)p.tile + 1]++;
+        o->most[w] = 0;
         for (int k = 0; k < pl.tiles(); ++k) {
-            c->res_most[w] = std::max(c->res_most[w], off[(size_t)k + 1]);
+            o->most[w] = std::max(o->most[w], off[(size_t)k + 1]);
             off[(size_t)k + 1] += off[k];
         }
-        c->res_off[w] = blk.size();
+        o->off[w] = blk.size();
         blk.insert(blk.end(), off.begin(), off.end());
-        c->res_own[w] = blk.size();
-        for (const Own &o : v) blk.push_back(o.own);
+        o->own[w] = blk.size();
+        for (const Own &p : v) blk.push_back(p.own);
         blk.resize((blk.size() + 1) / 2 * 2);  // entries are pairs
-        c->res_ent[w] = blk.size();
-        for (const Own &o : v) {
-            blk.push_back(o.kind << 24 | o.el);
-            blk.push_back(o.idx);
+        o->ent[w] = blk.size();
+        for (const Own &p : v) {
+            blk.push_back(p.kind << 24 | p.el);
+            blk.push_back(p.idx);
         }
     }
-    int rc;
-    if ((rc = c->regrow((void **)&c->res_lst, blk.size() * sizeof(int)))) return rc;
-    HIP_OK(h2d(c->stream, c->res_lst, blk.data(), blk.size() * sizeof(int)));
-    return DN_OK;
 }
-
-}  // namespace
 
 StepCtl dn::base_ctl(dn_ctx *c, int lv, int ls)
 {
@@ -446,10 +456,12 @@ int finish_run(dn_ctx *c, size_t nsample_events, bool *aborted = nullptr)
     return DN_OK;
 }
 
+}  // namespace
+
 // LDS of a run: the plan's, and the point lists (16-byte rounded)
-size_t res_lds(const dn_ctx *c, int sw)
+size_t dn::res_lds(const ResPlan &pl, const ResPoints &pt, int sw)
 {
-    return c->res.lds + (size_t)((c->res_most[2 * sw] + c->res_most[2 * sw + 1] + 1) & ~1) * sizeof(uint2);
+    return pl.lds + (size_t)((pt.most[2 * sw] + pt.most[2 * sw + 1] + 1) & ~1) * sizeof(uint2);
 }
 
 // Runs that the chip-resident loop takes: the grid fits (res_plan), a kernel
@@ -458,12 +470,10 @@ size_t res_lds(const dn_ctx *c, int sw)
 // land between launches), no CPML stretching (k_max_PML 1), no ux / uy / uxy output (GRAD_FORM 2 with
 // snapshots), no energy sums, wavefield snapshots or kernel sampling, and no
 // sweep shape or cache policy chosen by the caller.
-bool res_applies(const dn_ctx *c, int sw)
+bool dn::res_applies(const dn_ctx *c, int sw)
 {
     if (!c->res.ok || c->sweeps_chosen || !res_compiled(c->a.physics, c->p.L, sw)) return false;
-    if (!c->res_lst_ok[2 * sw] || !c->res_lst_ok[2 * sw + 1]) return false;
-    if (c->res_most[2 * sw] > RES_ENT || c->res_most[2 * sw + 1] > RES_ENT) return false;
-    if (res_lds(c, sw) > res_pool_lds(c->res_pool)) return false;
+    if (!c->res_pts.ok[2 * sw] || !c->res_pts.ok[2 * sw + 1]) return false;
     if (c->p.L > 0 && !c->tau_const) return false;  // relaxation times as planes
     // the curl at acoustic receivers differences vx along y and vy along x,
     // halo cells that the acoustic update does not need
@@ -477,16 +487,17 @@ bool res_applies(const dn_ctx *c, int sw)
     return c->p.dh >= 0x1p-60f && c->p.dh <= 0x1p60f;
 }
 
-// nsteps time steps from the zeroed state by the chip-resident loop.  *done
-// stays false when it did not run to its end (no free CUs, refused launch,
-// abandoned wait): the state is then undefined and the caller starts over.
-int res_run(dn_ctx *c, const StepCtl &ctl, int sw, int nsteps, bool *done)
+// the point lists of a plan fit beside its fields
+bool dn::res_points_fit(const dn_ctx *c, const ResPlan &pl, const ResPoints &pt, int sw)
 {
-    *done = false;
-    ResLease l;
-    ResPlan pl = c->res;
-    pl.lds = res_lds(c, sw);
-    if (!res_pool_take(c->res_pool, pl, nsteps, &l)) return DN_OK;
+    return pt.most[2 * sw] <= RES_ENT && pt.most[2 * sw + 1] <= RES_ENT &&
+           res_lds(pl, pt, sw) <= res_pool_lds(c->res_pool);
+}
+
+// launch arguments of nlast steps of a plan whose point lists are at lst;
+// mailboxes, tags and the steps of the launch are the caller's
+ResArgs dn::res_args(const dn_ctx *c, const ResPlan &pl, const ResPoints &pt, const int *lst, int sw, int nlast)
+{
     ResArgs r{};
     r.tw = pl.tw;
     r.th = pl.th;
@@ -499,30 +510,48 @@ int res_run(dn_ctx *c, const StepCtl &ctl, int sw, int nsteps, bool *done)
     r.cap = pl.cap;
     r.ncx = pl.ncx;
     r.ncy = pl.ncy;
-    r.nve = c->res_most[2 * sw];
-    r.nse = c->res_most[2 * sw + 1];
-    r.nlast = nsteps;
+    r.nve = pt.most[2 * sw];
+    r.nse = pt.most[2 * sw + 1];
+    r.nlast = nlast;
     r.fwdstore = c->p.mode > 0;
     r.dtinv = c->p.dtinv > 0 ? c->p.dtinv : 1;
     r.vp1_form = c->p.grad_form == 1 || c->p.grad_form == 2;
     r.rdh = 1.0 / (double)c->p.dh;
-    r.mbox = l.mbox;
-    r.abort = c->acq.nan_step + 1;
     const int v = 2 * sw, s = 2 * sw + 1;
-    r.voff = c->res_lst + c->res_off[v];
-    r.vown = c->res_lst + c->res_own[v];
-    r.vent = reinterpret_cast<const uint2 *>(c->res_lst + c->res_ent[v]);
-    r.soff = c->res_lst + c->res_off[s];
-    r.sown = c->res_lst + c->res_own[s];
-    r.sent = reinterpret_cast<const uint2 *>(c->res_lst + c->res_ent[s]);
+    r.voff = lst + pt.off[v];
+    r.vown = lst + pt.own[v];
+    r.vent = reinterpret_cast<const uint2 *>(lst + pt.ent[v]);
+    r.soff = lst + pt.off[s];
+    r.sown = lst + pt.own[s];
+    r.sent = reinterpret_cast<const uint2 *>(lst + pt.ent[s]);
+    return r;
+}
+
+namespace {
+
+// nsteps time steps from the zeroed state by the chip-resident loop.  *done
+// stays false when it did not run to its end (no free CUs, refused launch,
+// abandoned wait): the state is then undefined and the caller starts over.
+int res_run(dn_ctx *c, const StepCtl &ctl, int sw, int nsteps, bool *done)
+{
+    *done = false;
+    ResLease l;
+    ResPlan pl = c->res;
+    if (!res_points_fit(c, pl, c->res_pts, sw) ||
+        !res_pool_take(c->res_pool, pl.tiles(), (size_t)pl.tiles() * 2 * pl.cap, res_tags(nsteps), &l))
+        return DN_OK;
+    pl.lds = res_lds(pl, c->res_pts, sw);
+    ResKernel k{c->a, ctl, c->acq, res_args(c, pl, c->res_pts, c->res_lst, sw, nsteps), nullptr, nullptr};
+    k.r.mbox = l.mbox;
+    k.r.abort = c->acq.nan_step + 1;
     unsigned tag = l.tag0;
     bool ok = true;
     for (int n = 1; n <= nsteps && ok; n += RES_CHUNK) {
-        r.n0 = n;
-        r.n1 = std::min(n + RES_CHUNK - 1, nsteps);
-        r.tag0 = tag;
-        tag += (unsigned)(r.n1 - r.n0 + 2);
-        ok = res_launch(c->a, ctl, c->acq, r, pl, c->fdoh, sw, c->stream);
+        k.r.n0 = n;
+        k.r.n1 = std::min(n + RES_CHUNK - 1, nsteps);
+        k.r.tag0 = tag;
+        tag += (unsigned)(k.r.n1 - k.r.n0 + 2);
+        ok = res_launch(k, pl, pl.tiles(), c->fdoh, sw, c->stream);
     }
     bool aborted = !ok;
     const int rc = finish_run(c, 0, &aborted);

@@ -89,10 +89,8 @@ struct dn_ctx {
     ResPool *res_pool = nullptr;
     ResPlan res;
     bool sweeps_chosen = false;
-    int *res_lst = nullptr;  // one block: per list offsets, owners, entries
-    size_t res_off[4] = {}, res_own[4] = {}, res_ent[4] = {};  // positions in it (ints)
-    bool res_lst_ok[4] = {};
-    int res_most[4] = {};  // entries of a tile, at most
+    ResPoints res_pts;
+    int *res_lst = nullptr;  // res_pts.blk on the device
     // timing
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double run_ms = 0.0, v_ms = 0.0, s_ms = 0.0;
@@ -173,6 +171,12 @@ struct dn_ctx {
 
 
 namespace dn {
+// chip-resident runs (dn_api.hip)
+void res_points(const dn_ctx *c, const ResPlan &pl, ResPoints *o);
+size_t res_lds(const ResPlan &pl, const ResPoints &pt, int sw);
+bool res_applies(const dn_ctx *c, int sw);
+bool res_points_fit(const dn_ctx *c, const ResPlan &pl, const ResPoints &pt, int sw);
+ResArgs res_args(const dn_ctx *c, const ResPlan &pl, const ResPoints &pt, const int *lst, int sw, int nlast);
 // zero the wavefields, memory variables and CPML state of a shot
 int zero_state(dn_ctx *c);
 // sweep control with the cell lists lv (velocity) and ls (stress)

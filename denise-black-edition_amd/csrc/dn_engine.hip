@@ -10,6 +10,11 @@
 // launches; a shot that has reached its NT leaves its blocks idle until the
 // host detaches it.  Shots can be attached and detached between calls
 // (continuous batching); their state stays in their contexts.
+//
+// Shots whose grids fit are advanced by the chip-resident loop instead, many
+// of them in one launch (a round, plan_rounds below): their tiles share the
+// CUs, and a launch carries a whole run of steps.  The rounds of a run of
+// steps follow each other on the engine's stream, the sweeps after them.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -19,6 +24,7 @@
 #include <vector>
 
 #include "dn_ctx.h"
+#include "dn_sweep_common.h"
 
 using namespace dn;
 
@@ -28,7 +34,35 @@ struct Job {
     dn_ctx *ctx;
     int phase;  // 0 forward, 1 adjoint
     long base;  // engine clock before its first step
+    bool sweeps = false;  // its chip-resident run was abandoned
+    int round = -1;       // the round that carries it, -1: the sweeps
+    ResPlan plan;
+    ResPoints pts;
+    size_t lst = 0;  // position of its point lists (ints)
 };
+
+// a launch of the chip-resident loop: shots of one FD order, relaxation
+// count, direction and thread shape
+struct Round {
+    ResPlan shape;  // threads and LDS of the launch
+    std::vector<int> jobs;
+    int fdoh = 0, sw = 0, tiles = 0;
+    size_t words = 0, blk = 0;  // mailbox words, position of its workgroups
+};
+
+// Fewest steps of a run that the rounds carry: a launch loads and stores the
+// whole state of its shots.  Three 400x200 shots, runs of 8 steps: 14.7 us a
+// step (sweeps 25.5), 32 steps 8.7; one 2000x600 shot 24.7 (32.3) and 12.1.
+constexpr int RES_MIN_STEPS = 8;
+// Shots in the sweeps beside a round: while the sweeps' shots stay within
+// the last-level cache (about 4.5e6 cells) a million cells more cost them 10
+// us a step, and the round 4.4 + 7.4 us; past it they cost 20 us and more.
+// 1.1e6 cells beside 1.9e6 in the sweeps: 48.9 us with the round, 47.6
+// without; 0.34e6: 42.5 and 39.4.  Beside 5.0e6: 83.3 and 108.1; 78.4 and 86.3.
+constexpr long RES_LLC_CELLS = 4500000;
+constexpr long RES_MIN_CELLS[2] = {1100000, 350000};  // of a round, within the cache and past it
+// LDS kept for the point lists of a tile
+constexpr size_t RES_PTS_LDS = 2048;
 
 struct Group {
     int fdoh, L, sw;
@@ -45,7 +79,7 @@ struct dn_engine {
     hipStream_t stream = nullptr;
     std::vector<Job> jobs;              // running shots
     std::map<dn_ctx *, int> status;     // last known state per shot
-    int *d_clock = nullptr;             // device clock (steps run)
+    int *d_clock = nullptr;             // device clock (steps run), abort word of the rounds
     long clock = 0;                     // its value once the queued work is done
     bool inflight = false;              // a launched run not yet waited for
     bool dirty = true;
@@ -57,6 +91,16 @@ struct dn_engine {
     int graph_steps = 0;
     hipGraphExec_t gexec = nullptr;
     hipGraph_t graph = nullptr;
+    // chip-resident rounds
+    ResPool *pool = nullptr;
+    std::vector<Round> rounds;
+    bool resident = false;  // the sweeps' tables leave the shots of the rounds out
+    bool leased = false;    // a launched run holds mailboxes and CUs
+    ResLease lease;
+    int *d_lst = nullptr;  // point lists
+    ResBlock *d_rblk = nullptr;
+    ResKernel *d_rtab = nullptr;
+    size_t cap_lst = 0, cap_rblk = 0, cap_rtab = 0;
 
     void drop_graph()
     {
@@ -73,19 +117,237 @@ struct dn_engine {
         if (d_clock) (void)hipFree(d_clock);
         if (d_shots) (void)hipFree(d_shots);
         if (d_blk) (void)hipFree(d_blk);
+        if (d_lst) (void)hipFree(d_lst);
+        if (d_rblk) (void)hipFree(d_rblk);
+        if (d_rtab) (void)hipFree(d_rtab);
+        if (leased) res_pool_give(pool, lease);
+        res_pool_close(pool);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
 
 namespace {
 
-// group every running shot and upload the launch tables
-int rebuild(dn_engine *e)
+// a device buffer of at least n elements; the old contents are lost
+template <class T>
+int grow(T **p, size_t *cap, size_t n)
+{
+    if (n <= *cap) return DN_OK;
+    if (*p) HIP_OK(hipFree(*p));
+    *p = nullptr;
+    const size_t c = std::max(n, 2 * *cap);
+    *cap = 0;
+    HIP_OK(hipMalloc((void **)p, sizeof(T) * c));
+    *cap = c;
+    return DN_OK;
+}
+
+// Which shots the chip-resident loop carries, and the rounds it does so in.
+// A round takes about 4.4 us a step and 1.9 us per thousand cells of a tile
+// (FDORDER 8, elastic: 340 cells 5.0 us, 4690 cells 13.3), so the fewest win:
+// shots are packed largest first by the fewest tiles that hold them, and the
+// CUs left over are then dealt out in proportion.
+int plan_rounds(dn_engine *e)
+{
+    e->rounds.clear();
+    for (Job &j : e->jobs) j.round = -1;
+    if (!e->pool) return DN_OK;
+    const int ncu = res_pool_cus(e->pool);
+    const size_t lds = res_pool_lds(e->pool) - RES_PTS_LDS;
+    struct Fit {
+        int job, least, need[RES_SHAPES];  // tiles by shape, 0: does not fit
+    };
+    std::map<std::tuple<int, int, int>, std::vector<Fit>> by;
+    long swept = 0;  // cells of the shots left to the sweeps
+    for (int k = 0; k < (int)e->jobs.size(); ++k) {
+        const Job &j = e->jobs[k];
+        Fit f{k, 0, {}};
+        if (!j.sweeps && res_applies(j.ctx, j.phase))
+            for (int s = 0; s < RES_SHAPES; ++s) {
+                const ResPlan pl = res_least(j.ctx->p, lds, s);
+                f.need[s] = pl.ok && pl.tiles() <= ncu ? pl.tiles() : 0;
+                if (f.need[s] && (!f.least || f.need[s] < f.least)) f.least = f.need[s];
+            }
+        if (f.least)
+            by[std::make_tuple(j.ctx->fdoh, j.ctx->p.L, j.phase)].push_back(f);
+        else
+            swept += (long)j.ctx->p.nx * j.ctx->p.ny;
+    }
+    struct Pack {
+        std::vector<Fit> fit;
+        int shape;
+        long cells;
+    };
+    // the lightest shape in which all shots of a round fit together, or -1
+    auto shape_of = [&](const std::vector<Fit> &v) {
+        for (int s = 0; s < RES_SHAPES; ++s) {
+            int sum = 0;
+            bool ok = true;
+            for (const Fit &f : v) {
+                ok = ok && f.need[s];
+                sum += f.need[s];
+            }
+            if (ok && sum <= ncu) return s;
+        }
+        return -1;
+    };
+    std::vector<Pack> packs;
+    for (auto &kv : by) {
+        auto &v = kv.second;
+        std::stable_sort(v.begin(), v.end(), [](const Fit &x, const Fit &y) { return x.least > y.least; });
+        const size_t first = packs.size();
+        for (const Fit &f : v) {
+            size_t k = first;
+            for (; k < packs.size(); ++k) {
+                std::vector<Fit> with = packs[k].fit;
+                with.push_back(f);
+                const int s = shape_of(with);
+                if (s < 0) continue;
+                packs[k].fit.swap(with);
+                packs[k].shape = s;
+                break;
+            }
+            if (k == packs.size()) packs.push_back(Pack{{f}, shape_of({f}), 0});
+        }
+    }
+    for (Pack &p : packs)
+        for (const Fit &f : p.fit) p.cells += (long)e->jobs[f.job].ctx->p.nx * e->jobs[f.job].ctx->p.ny;
+    std::stable_sort(packs.begin(), packs.end(), [](const Pack &x, const Pack &y) { return x.cells < y.cells; });
+    for (const Pack &p : packs) {
+        if (swept && p.cells < RES_MIN_CELLS[swept + p.cells > RES_LLC_CELLS]) {
+            swept += p.cells;
+            continue;
+        }
+        Round r;
+        int sum = 0;
+        for (const Fit &f : p.fit) sum += f.need[p.shape];
+        for (const Fit &f : p.fit) {
+            Job &j = e->jobs[f.job];
+            const ResPlan pl = res_plan(j.ctx->p, (int)((long)ncu * f.need[p.shape] / sum), lds, p.shape);
+            if (!pl.ok) continue;
+            res_points(j.ctx, pl, &j.pts);
+            if (!res_points_fit(j.ctx, pl, j.pts, j.phase)) continue;
+            j.plan = pl;
+            j.round = (int)e->rounds.size();
+            if (r.jobs.empty()) r.shape = pl;
+            r.shape.nthr = std::max(r.shape.nthr, pl.nthr);
+            r.shape.lds = std::max(r.shape.lds, res_lds(pl, j.pts, j.phase));
+            r.fdoh = j.ctx->fdoh;
+            r.sw = j.phase;
+            r.tiles += pl.tiles();
+            r.words += (size_t)pl.tiles() * 2 * pl.cap;
+            r.jobs.push_back(f.job);
+        }
+        if (!r.jobs.empty()) e->rounds.push_back(r);
+    }
+    // their point lists and workgroups; neighbouring tiles share an XCD's L2
+    std::vector<int> lst;
+    std::vector<ResBlock> blk;
+    int slot = 0;
+    for (Round &r : e->rounds) {
+        std::vector<ResBlock> v;
+        for (int k : r.jobs) {
+            Job &j = e->jobs[k];
+            lst.resize((lst.size() + 1) / 2 * 2);
+            j.lst = lst.size();
+            lst.insert(lst.end(), j.pts.blk.begin(), j.pts.blk.end());
+            for (int t = 0; t < j.plan.tiles(); ++t) v.push_back(ResBlock{slot, t});
+            ++slot;
+        }
+        r.blk = blk.size();
+        for (int b = 0; b < r.tiles; ++b) blk.push_back(v[(size_t)xcd_tile(b, r.tiles)]);
+    }
+    if (e->rounds.empty()) return DN_OK;
+    int rc;
+    if ((rc = grow(&e->d_lst, &e->cap_lst, lst.size())) || (rc = grow(&e->d_rblk, &e->cap_rblk, blk.size()))) return rc;
+    HIP_OK(h2d(e->stream, e->d_lst, lst.data(), lst.size() * sizeof(int)));
+    HIP_OK(h2d(e->stream, e->d_rblk, blk.data(), blk.size() * sizeof(ResBlock)));
+    return DN_OK;
+}
+
+// the rounds of `steps` steps from the engine's clock
+int launch_rounds(dn_engine *e, int steps)
+{
+    const int parts = (steps + RES_CHUNK - 1) / RES_CHUNK;
+    std::vector<ResKernel> tab;
+    unsigned tag = e->lease.tag0;
+    for (const Round &r : e->rounds)
+        for (int part = 0; part < parts; ++part) {
+            res_word *box = e->lease.mbox;
+            const int k0 = part * RES_CHUNK, k1 = std::min(k0 + RES_CHUNK, steps);  // of this run
+            for (int k : r.jobs) {
+                const Job &j = e->jobs[k];
+                dn_ctx *c = j.ctx;
+                StepCtl ctl = j.phase == 0 ? base_ctl(c, 0, 1) : base_ctl(c, 2, 3);
+                ctl.seismo = j.phase == 0 ? c->p.seismo : 0;
+                ctl.probe = 1;
+                ResPlan pl = j.plan;
+                pl.nk_s = pl.nk_v = (pl.cap + r.shape.nthr - 1) / r.shape.nthr;
+                ResKernel a{c->a, ctl, c->acq, res_args(c, pl, j.pts, e->d_lst + j.lst, j.phase, c->p.nt), nullptr, nullptr};
+                a.r.mbox = box;
+                a.r.abort = e->d_clock + 1;
+                a.r.tag0 = tag;
+                a.r.n0 = (int)(e->clock - j.base) + k0;
+                a.r.n1 = std::min((int)(e->clock - j.base) + k1 - 1, c->p.nt);
+                box += (size_t)pl.tiles() * 2 * pl.cap;
+                tab.push_back(a);
+            }
+            tag += (unsigned)(k1 - k0 + 2);
+        }
+    int rc;
+    if ((rc = grow(&e->d_rtab, &e->cap_rtab, tab.size()))) return rc;
+    HIP_OK(h2d(e->stream, e->d_rtab, tab.data(), tab.size() * sizeof(ResKernel)));
+    size_t at = 0;
+    int slot = 0;  // of the round's first shot in the workgroups' table
+    for (const Round &r : e->rounds) {
+        for (int part = 0; part < parts; ++part) {
+            ResKernel k = tab[at];
+            k.tab = e->d_rtab + at - slot;
+            k.blk = e->d_rblk + r.blk;
+            if (!res_launch(k, r.shape, r.tiles, r.fdoh, r.sw, e->stream)) {
+                // the rounds already launched run to their end: every shot of
+                // the rounds starts over, as after an abandoned wait
+                static const int one = 1;
+                HIP_OK(h2d(e->stream, e->d_clock + 1, &one, sizeof(int)));
+                return DN_OK;
+            }
+            at += r.jobs.size();
+        }
+        slot += (int)r.jobs.size();
+    }
+    return DN_OK;
+}
+
+// a shot's state before its first step
+int begin_shot(dn_ctx *c, int phase)
+{
+    int rc;
+    if ((rc = zero_state(c))) return rc;
+    if (phase == 1) {
+        const size_t g = (size_t)c->p.nx * c->p.ny * sizeof(float);
+        HIP_OK(hipMemsetAsync(c->wc, 0, g, c->stream));
+        HIP_OK(hipMemsetAsync(c->wcu, 0, g, c->stream));
+        HIP_OK(hipMemsetAsync(c->wcr, 0, g, c->stream));
+    } else {
+        c->fwd_complete = false;
+        // grad_obj_psv.c:71-76: the energies start at zero for each shot
+        if (c->eprecond)
+            for (int w = 0; w < 2; ++w)
+                HIP_OK(hipMemsetAsync(c->ew[w], 0, (size_t)c->p.nx * c->p.ny * sizeof(float), c->stream));
+    }
+    HIP_OK(hipStreamSynchronize(c->stream));
+    return DN_OK;
+}
+
+// group the running shots (resident: those no round carries) and upload the
+// launch tables of the sweeps
+int rebuild(dn_engine *e, bool resident)
 {
     HIP_OK(hipStreamSynchronize(e->stream));
     e->drop_graph();
     std::map<std::tuple<int, int, int, int, int, int, int, int, int, int, int>, std::vector<int>> by;
     for (int k = 0; k < (int)e->jobs.size(); ++k) {
+        if (resident && e->jobs[k].round >= 0) continue;
         const dn_ctx *c = e->jobs[k].ctx;
         const Tile &v = c->tile_v, &s = c->tile_s;
         by[std::make_tuple(c->fdoh, c->p.L, e->jobs[k].phase, v.tbx, v.by, v.ty, v.vw, s.tbx, s.by, s.ty, s.vw)]
@@ -161,6 +423,7 @@ int rebuild(dn_engine *e)
     if (!shots.empty()) HIP_OK(h2d(e->stream, e->d_shots, shots.data(), sizeof(BatchShot) * shots.size()));
     if (!blk.empty()) HIP_OK(h2d(e->stream, e->d_blk, blk.data(), sizeof(BatchBlock) * blk.size()));
     e->n_shots = (int)shots.size();
+    e->resident = resident;
     e->dirty = false;
     return DN_OK;
 }
@@ -227,12 +490,13 @@ int dn_engine_create(int device, dn_engine **out)
         delete e;
         return fail(DN_ERR_HIP, "stream creation failed");
     }
-    const int zero = 0;
-    if (hipMalloc((void **)&e->d_clock, sizeof(int)) != hipSuccess ||
-        h2d(e->stream, e->d_clock, &zero, sizeof(int)) != hipSuccess) {
+    const int zero[2] = {0, 0};
+    if (hipMalloc((void **)&e->d_clock, sizeof zero) != hipSuccess ||
+        h2d(e->stream, e->d_clock, zero, sizeof zero) != hipSuccess) {
         delete e;
         return fail(DN_ERR_OOM, "engine clock");
     }
+    e->pool = res_pool_open(device);
     *out = e;
     return DN_OK;
 }
@@ -266,29 +530,23 @@ int dn_engine_attach(dn_engine *e, dn_ctx *c, int phase)
         return fail(DN_ERR_STATE, "adjoint phase needs a finished forward phase with snapshots");
     if (e->clock > (1L << 30)) return fail(DN_ERR_STATE, "engine clock exhausted; create a new engine");
     HIP_OK(hipSetDevice(e->device));
-    // tile shapes the multi-shot kernels are compiled for
+    // tile shapes the multi-shot kernels are compiled for; the caller did not
+    // choose them
     int rc;
+    const bool chosen = c->sweeps_chosen;
     if (!batch_tile_supported(c->tile_v, 0) && (rc = dn_set_tile(c, 0, 128, 2, 4, 1))) return rc;
     // (elastic groups default to 64,4,2,2: on the 64-shot mix 50.7 Gcell/s
     // against 49.2 with 64,4,1,4 and 42.2 with 64,4,2,1)
     if ((!batch_str_supported(c->tile_s, c->p.L) || (c->p.L == 0 && c->tile_s.ty == 1 && c->tile_s.vw == 1)) &&
         (rc = c->p.L == 0 ? dn_set_tile(c, 1, 64, 4, 2, 2) : dn_set_tile(c, 1, 64, 4, 1, 1)))
         return rc;
-    if ((rc = zero_state(c))) return rc;
-    if (phase == 1) {
-        const size_t g = (size_t)c->p.nx * c->p.ny * sizeof(float);
-        HIP_OK(hipMemsetAsync(c->wc, 0, g, c->stream));
-        HIP_OK(hipMemsetAsync(c->wcu, 0, g, c->stream));
-        HIP_OK(hipMemsetAsync(c->wcr, 0, g, c->stream));
-    } else {
-        c->fwd_complete = false;
-        // grad_obj_psv.c:71-76: the energies start at zero for each shot
-        if (c->eprecond)
-            for (int w = 0; w < 2; ++w)
-                HIP_OK(hipMemsetAsync(c->ew[w], 0, (size_t)c->p.nx * c->p.ny * sizeof(float), c->stream));
-    }
-    HIP_OK(hipStreamSynchronize(c->stream));
-    e->jobs.push_back(Job{c, phase, e->clock - 1});
+    c->sweeps_chosen = chosen;
+    if ((rc = begin_shot(c, phase))) return rc;
+    Job j;
+    j.ctx = c;
+    j.phase = phase;
+    j.base = e->clock - 1;
+    e->jobs.push_back(j);
     e->status[c] = 1;
     e->dirty = true;
     return DN_OK;
@@ -300,20 +558,38 @@ int dn_engine_launch(dn_engine *e, int nsteps)
     if (e->inflight) return fail(DN_ERR_STATE, "a launched run is still in flight (dn_engine_wait first)");
     HIP_OK(hipSetDevice(e->device));
     int rc;
-    const bool changed = e->dirty;
-    if (changed && (rc = rebuild(e))) return rc;
+    // a shot that the loop no longer takes (its options were changed) leaves its round
+    for (const Job &j : e->jobs)
+        if (j.round >= 0 && !res_applies(j.ctx, j.phase)) e->dirty = true;
     if (e->jobs.empty() || nsteps == 0) return DN_OK;
+    if (e->dirty && (rc = plan_rounds(e))) return rc;
     // no more steps than the longest remaining shot needs
     long need = 0;
     for (const Job &j : e->jobs) need = std::max<long>(need, j.ctx->p.nt - (e->clock - j.base) + 1);
     int left = (int)std::min<long>(nsteps, need);
-    e->clock += left;
+    bool resident = !e->rounds.empty() && left >= RES_MIN_STEPS;
+    if (resident) {
+        int tiles = 0;
+        size_t words = 0;
+        for (const Round &r : e->rounds) {
+            tiles = std::max(tiles, r.tiles);
+            words = std::max(words, r.words);
+        }
+        // (every launch draws its own tags)
+        const unsigned long tags = (unsigned long)res_tags(left) * e->rounds.size();
+        e->leased = tags < 0x7fffffffUL && res_pool_take(e->pool, tiles, words, (unsigned)tags, &e->lease);
+        resident = e->leased;
+    }
+    const bool changed = e->dirty || resident != e->resident;
     e->inflight = true;
+    if (changed && (rc = rebuild(e, resident))) return rc;
+    if (resident && (rc = launch_rounds(e, left))) return rc;
+    e->clock += left;
     // a graph is captured only for a set of shots that has already run
     // unchanged once: capture and instantiation cost milliseconds of host
     // time, which a set that changes at every call (a request stream) would
     // pay each time while plain launches overlap the GPU work
-    if (e->graph_steps > 0 && left >= e->graph_steps && (e->gexec || !changed)) {
+    if (e->graph_steps > 0 && left >= e->graph_steps && (e->gexec || !changed) && !e->groups.empty()) {
         if (!e->gexec && (rc = capture(e))) return rc;
         for (; left >= e->graph_steps; left -= e->graph_steps) HIP_OK(hipGraphLaunch(e->gexec, e->stream));
     }
@@ -330,6 +606,25 @@ int dn_engine_wait(dn_engine *e, int *running)
         e->inflight = false;
         HIP_OK(hipStreamSynchronize(e->stream));
         int rc;
+        if (e->leased) {
+            res_pool_give(e->pool, e->lease);
+            e->leased = false;
+            int word[2] = {0, 0};
+            HIP_OK(d2h(e->stream, word, e->d_clock, sizeof word));
+            if (word[1]) {
+                // the workgroups gave up waiting for each other: the shots of
+                // the rounds start over, in the sweeps
+                word[1] = 0;
+                HIP_OK(h2d(e->stream, e->d_clock + 1, word + 1, sizeof(int)));
+                for (Job &j : e->jobs) {
+                    if (j.round < 0) continue;
+                    if ((rc = begin_shot(j.ctx, j.phase))) return rc;
+                    j.sweeps = true;
+                    j.base = e->clock - 1;
+                }
+                e->dirty = true;
+            }
+        }
         if ((rc = collect(e))) return rc;
     }
     if (running) *running = (int)e->jobs.size();

@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 #include "dn_resident_plan.h"
 
 namespace dn {
@@ -23,19 +25,35 @@ struct ResArgs {
     const uint2 *vent, *sent;
 };
 
-// the kernel's one argument
+// the point lists of a plan, one block: per list offsets, owners, entries
+struct ResPoints {
+    std::vector<int> blk;
+    size_t off[4] = {}, own[4] = {}, ent[4] = {};  // positions in it (ints)
+    bool ok[4] = {};   // no point that the loop has no place for
+    int most[4] = {};  // entries of a tile, at most
+};
+
+// one workgroup of a launch that holds several shots
+struct ResBlock {
+    int shot, tile;
+};
+
+// the kernel's one argument: a shot, or the shots of the launch (tab) and
+// the shot and tile of every workgroup (blk)
 struct ResKernel {
     KArgs a;
     StepCtl c;
     DevAcq q;
     ResArgs r;
+    const ResKernel *tab;
+    const ResBlock *blk;
 };
 
 // is there a compiled kernel for this run (sw 0 forward, 1 adjoint)
 bool res_compiled(int physics, int L, int sw);
-// enqueue one launch; false when the runtime refuses it
-bool res_launch(const KArgs &a, const StepCtl &c, const DevAcq &q, const ResArgs &r, const ResPlan &pl, int fdoh,
-                int sw, void *stream);
+// enqueue one launch of as many workgroups, with the threads, LDS and thread
+// shape of pl; false when the runtime refuses it
+bool res_launch(const ResKernel &k, const ResPlan &pl, int blocks, int fdoh, int sw, void *stream);
 
 // The mailboxes of a device: one allocation shared by the contexts on it,
 // made with the first and given back with the last, and the account of its
@@ -49,11 +67,14 @@ ResPool *res_pool_open(int device);  // nullptr: no pool (no memory)
 void res_pool_close(ResPool *p);
 int res_pool_cus(const ResPool *p);
 size_t res_pool_lds(const ResPool *p);
+// step tags of a run: one for each step and two for each launch
+constexpr unsigned res_tags(int steps) { return (unsigned)steps + 2u * (unsigned)(steps / RES_CHUNK + 2); }
 struct ResLease {
     res_word *mbox = nullptr;
     unsigned tag0 = 0;
 };
-bool res_pool_take(ResPool *p, const ResPlan &pl, int steps, ResLease *out);
+// mailboxes of so many words, CUs for so many tiles, and step tags
+bool res_pool_take(ResPool *p, int tiles, size_t words, unsigned tags, ResLease *out);
 void res_pool_give(ResPool *p, const ResLease &l);
 
 }  // namespace dn

@@ -10,18 +10,16 @@
 namespace dn {
 
 template <int F, int GROUP>
-bool res_launch_f(const KArgs &a, const StepCtl &c, const DevAcq &q, const ResArgs &r, const ResPlan &pl, int sw,
-                  hipStream_t s);
+bool res_launch_f(const ResKernel &k, const ResPlan &pl, int blocks, int sw, hipStream_t s);
 
-bool res_launch(const KArgs &a, const StepCtl &c, const DevAcq &q, const ResArgs &r, const ResPlan &pl, int fdoh,
-                int sw, void *stream)
+bool res_launch(const ResKernel &k, const ResPlan &pl, int blocks, int fdoh, int sw, void *stream)
 {
     hipStream_t s = (hipStream_t)stream;
-#define DN_F(F)                                                      \
-    case F:                                                          \
-        return a.physics != 1 ? res_launch_f<F, 1>(a, c, q, r, pl, sw, s) \
-               : a.L > 0      ? res_launch_f<F, 2>(a, c, q, r, pl, sw, s) \
-                              : res_launch_f<F, 0>(a, c, q, r, pl, sw, s);
+#define DN_F(F)                                                                \
+    case F:                                                                    \
+        return k.a.physics != 1 ? res_launch_f<F, 1>(k, pl, blocks, sw, s) \
+               : k.a.L > 0      ? res_launch_f<F, 2>(k, pl, blocks, sw, s) \
+                                : res_launch_f<F, 0>(k, pl, blocks, sw, s);
     switch (fdoh) {
         DN_F(1) DN_F(2) DN_F(3) DN_F(4) DN_F(5) DN_F(6)
     }
@@ -58,7 +56,7 @@ bool clear(ResPool *p)
 {
     hipStream_t s = nullptr;
     const bool ok = hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess &&
-                    hipMemsetAsync(p->mem, 0, p->words * sizeof(res_word), s) == hipSuccess &&
+                    hipMemsetAsync(p->mem, 0, (p->words + 1024) * sizeof(res_word), s) == hipSuccess &&
                     hipStreamSynchronize(s) == hipSuccess;
     if (s) (void)hipStreamDestroy(s);
     if (ok)
@@ -89,8 +87,9 @@ ResPool *res_pool_open(int device)
     q->device = device;
     q->ncu = ncu;
     q->lds = (size_t)lds;
+    // (a workgroup reads past its last words, at most a word per thread)
     q->words = (size_t)ncu * 2 * RES_CAP;
-    if (hipMalloc((void **)&q->mem, q->words * sizeof(res_word)) != hipSuccess || !clear(q)) {
+    if (hipMalloc((void **)&q->mem, (q->words + 1024) * sizeof(res_word)) != hipSuccess || !clear(q)) {
         (void)hipGetLastError();
         if (q->mem) (void)hipFree(q->mem);
         delete q;
@@ -114,11 +113,10 @@ void res_pool_close(ResPool *p)
 int res_pool_cus(const ResPool *p) { return p->ncu; }
 size_t res_pool_lds(const ResPool *p) { return p->lds; }
 
-bool res_pool_take(ResPool *p, const ResPlan &pl, int steps, ResLease *out)
+bool res_pool_take(ResPool *p, int tiles, size_t words, unsigned tags, ResLease *out)
 {
     std::lock_guard<std::mutex> g(p->m);
-    if (p->tiles + pl.tiles() > p->ncu) return false;
-    const size_t words = (size_t)pl.tiles() * 2 * pl.cap;
+    if (p->tiles + tiles > p->ncu) return false;
     size_t at = 0, k = 0;
     for (; k < p->busy.size(); ++k) {  // first gap
         if (p->busy[k].at - at >= words) break;
@@ -128,12 +126,12 @@ bool res_pool_take(ResPool *p, const ResPlan &pl, int steps, ResLease *out)
     // tags must not come round again over words that hold them: an idle pool
     // half way through them starts afresh
     if (p->busy.empty() && p->next > 0x80000000u && !clear(p)) return false;
-    if (p->next > 0xffffffffu - (unsigned)steps - 2u * (unsigned)(steps / RES_CHUNK + 2)) return false;
+    if (tags > 0x7fffffffu || p->next > 0xffffffffu - tags) return false;
     out->mbox = p->mem + at;
     out->tag0 = p->next;
-    p->next += (unsigned)steps + 2u * (unsigned)(steps / RES_CHUNK + 2);
-    p->busy.insert(p->busy.begin() + (long)k, ResPool::Range{at, words, pl.tiles()});
-    p->tiles += pl.tiles();
+    p->next += tags;
+    p->busy.insert(p->busy.begin() + (long)k, ResPool::Range{at, words, tiles});
+    p->tiles += tiles;
     return true;
 }
 

@@ -54,8 +54,14 @@ struct ResPlan {
 inline int res_planes(int physics) { return physics == 2 || physics == 5 ? 3 : 5; }
 
 // the plan of a grid on a device with ncu CUs and lds_max bytes of LDS per
-// workgroup (ok = false: the grid does not fit)
-ResPlan res_plan(const dn_params &p, int ncu, size_t lds_max);
+// workgroup (ok = false: the grid does not fit); shape: one entry of
+// res_shapes, or -1 for the lightest that fits
+ResPlan res_plan(const dn_params &p, int ncu, size_t lds_max, int shape = -1);
+// the plan of that shape with the fewest tiles
+ResPlan res_least(const dn_params &p, size_t lds_max, int shape);
+// rows and columns per thread, from the lightest
+constexpr int RES_SHAPES = 5;
+constexpr int res_shapes[RES_SHAPES][2] = {{1, 1}, {1, 2}, {1, 4}, {2, 4}, {3, 4}};
 // LDS planes: vx, vy and the stresses (acoustic: vx, vy, p; SH: vz, sxz, syz)
 enum { PL_VX = 0, PL_VY = 1, PL_SXX = 2, PL_SYY = 3, PL_SXY = 4 };
 enum { PL_P = 2 };

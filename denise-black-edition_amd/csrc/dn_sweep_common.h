@@ -19,7 +19,7 @@ __device__ __forceinline__ float cpml(float &psi, float b, float a, float K, flo
 // Block -> tile: workgroups are dispatched to the XCDs round-robin, so the
 // blocks of XCD x are x, x+8, x+16, ...; give them the contiguous tile range
 // [start_x, start_x + count_x).
-__device__ __forceinline__ int xcd_tile(int bid, int ntiles)
+__host__ __device__ __forceinline__ int xcd_tile(int bid, int ntiles)
 {
     const int per = ntiles / NXCD, rem = ntiles % NXCD;
     const int x = bid % NXCD, k = bid / NXCD;

@@ -147,6 +147,36 @@ static bool one(dn_params p)
     return true;
 }
 
+// the plans of a launch that holds several grids: a given thread shape in few
+// tiles, with the threads of the launch's largest workgroup
+template <int F, int PH>
+static int packed(dn_params p)
+{
+    p.physics = PH;
+    p.fdorder = 2 * F;
+    int n = 0;
+    for (int s = 0; s < RES_SHAPES; ++s) {
+        const ResPlan least = res_least(p, 163840 - 2048, s);
+        if (!least.ok || least.tiles() > 256) continue;
+        // no thread shape and budget below it fits
+        CHECK(!res_plan(p, least.tiles() - 1, 163840 - 2048, s).ok);
+        for (int more : {0, 7}) {
+            ResPlan pl = res_plan(p, least.tiles() + more, 163840 - 2048, s);
+            CHECK(pl.ok && pl.tiles() <= least.tiles() + more);
+            CHECK(pl.ry == res_shapes[s][0] && pl.vx == res_shapes[s][1]);
+            if (more) {
+                pl.nthr = std::min(pl.nthr + 128, res_maxt(pl.ry, pl.vx, F, p.L));
+                pl.nk_s = pl.nk_v = (pl.cap + pl.nthr - 1) / pl.nthr;
+            }
+            if (pl.ry == 1) check<F, PH, res_width(1)>(p, pl);
+            if (pl.ry == 2) check<F, PH, res_width(2)>(p, pl);
+            if (pl.ry == 3) check<F, PH, res_width(3)>(p, pl);
+            ++n;
+        }
+    }
+    return n;
+}
+
 template <int F>
 static int orders(const dn_params &p)
 {
@@ -178,6 +208,14 @@ int main()
         p.fw = std::min(10, std::min(p.nx, p.ny) / 2);
         p.free_surf = k % 2;
         fit += orders<2>(p) + orders<4>(p) + orders<5>(p);
+    }
+    for (int k = 0; k < 5; ++k) {
+        dn_params p{};
+        p.nx = 60 + (int)(rng() % 700);
+        p.ny = 40 + (int)(rng() % 300);
+        p.fw = 10;
+        p.free_surf = k % 2;
+        fit += packed<2, 1>(p) + packed<4, 1>(p);
     }
     std::printf("%s, %d plans\n", fails ? "resident geometry wrong" : "resident geometry ok", fit);
     return fails ? 1 : 0;

@@ -183,3 +183,63 @@ def test_concurrent_contexts():
     for t in ts:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("steps", [[200], [40, 3, 17, 5, 9, 200]])
+@pytest.mark.parametrize("large", [False, True])
+def test_engine_rounds_equal_sweeps(steps, large):
+    """Shots of several orders, sizes, lengths and relaxation counts together
+    (the loop's rounds, large: and a grid for the sweeps, which the small
+    rounds join), runs of steps that move them between the loop and the
+    sweeps, and a shot that joins on the way."""
+    sizes = [(131, 77, 90, 8, 0), (611, 303, 70, 8, 0), (1003, 401, 50, 8, 0), (29, 21, 130, 8, 0), (733, 290, 80, 4, 0),
+             (260, 120, 60, 4, 1), (320, 200, 75, 8, 2), (210, 90, 40, 12, 3)]
+    if large:
+        sizes += [(1301, 801, 40, 8, 0), (2600, 900, 30, 8, 0)]
+    cases = [make_case(nx=nx, ny=ny, nt=nt, fdorder=o, L=L, fw=5 if ny < 40 else 10, seismo=4, homogeneous=True,
+                       nrec=nx // 3, seed=k + 1) for k, (nx, ny, nt, o, L) in enumerate(sizes)]
+    eng = dnhip.Engine()
+    shots = [context(c, False) for c in cases]
+    for g in shots[1:]:
+        eng.attach(g)
+    print("rounds of chip-resident shots", flush=True)
+    for k, n in enumerate(steps):
+        eng.step(n)
+        if k == 0:
+            eng.attach(shots[0])
+    eng.run()
+    for case, g in zip(cases, shots):
+        assert eng.status(g) == 0
+        ref = context(case, True)
+        ref.forward()
+        assert np.abs(ref.field(dnhip.F_VX)).max() > 0
+        for k, (x, y) in enumerate(zip(state(g, case[0]), state(ref, case[0]))):
+            np.testing.assert_array_equal(x, y, err_msg=f"{case[0].nx}x{case[0].ny} output {k}")
+
+
+def test_engine_gradient_rounds_equal_sweeps():
+    """Forward and adjoint phases of two grids in the engine's rounds."""
+    cases = [make_case(nx=nx, ny=ny, nt=120, fw=10, mode=1, dtinv=2, fc=15.0, nrec=nx // 4, seed=nx)
+             for nx, ny in [(333, 150), (905, 411)]]
+    eng = dnhip.Engine()
+    for chunk in (16, 200):
+        shots = [context(c, False) for c in cases]
+        for g in shots:
+            eng.attach(g, 0)
+        eng.run(chunk)
+        for g in shots:
+            zero = np.zeros_like(g.seismogram(0))
+            g.residuals(zero, zero, None, 1)
+            eng.attach(g, 1)
+        print("gradient rounds", flush=True)
+        eng.run(chunk)
+        for case, g in zip(cases, shots):
+            ref = context(case, True)
+            ref.forward()
+            zero = np.zeros_like(ref.seismogram(0))
+            ref.residuals(zero, zero, None, 1)
+            ref.adjoint()
+            g.assemble()
+            ref.assemble()
+            for w in range(6):
+                np.testing.assert_array_equal(g.gradient(w), ref.gradient(w), err_msg=f"{case[0].nx} gradient {w}")
