@@ -15,6 +15,10 @@
 // of them in one launch (a round, plan_rounds below): their tiles share the
 // CUs, and a launch carries a whole run of steps.  The rounds of a run of
 // steps follow each other on the engine's stream, the sweeps after them.
+//
+// The sweeps' groups, too, need not advance together: each goes through the
+// whole run of steps before the next, and a group whose wavefields and
+// materials exceed the last-level cache is cut into several that do not.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -56,11 +60,12 @@ struct Round {
 constexpr int RES_MIN_STEPS = 8;
 // Shots in the sweeps beside a round: while the sweeps' shots stay within
 // the last-level cache (about 4.5e6 cells) a million cells more cost them 10
-// us a step, and the round 4.4 + 7.4 us; past it they cost 20 us and more.
-// 1.1e6 cells beside 1.9e6 in the sweeps: 48.9 us with the round, 47.6
-// without; 0.34e6: 42.5 and 39.4.  Beside 5.0e6: 83.3 and 108.1; 78.4 and 86.3.
+// us a step, and the round 4.4 + 7.4 us; past it they need another 14 us.
+// 1.1e6 cells beside 1.9e6 in the sweeps: 48.9 us with the round, 47.7
+// without; 0.34e6: 42.5 and 38.8.  Beside 5.0e6: 1.1e6 81.4 and 96.1, 0.79e6
+// 79.7 and 89.7; beside 7.8e6: 1.1e6 119.5 and 119.5, 0.34e6 142.6 and 110.2.
 constexpr long RES_LLC_CELLS = 4500000;
-constexpr long RES_MIN_CELLS[2] = {1100000, 350000};  // of a round, within the cache and past it
+constexpr long RES_MIN_CELLS[2] = {1100000, 700000};  // of a round, within the cache and past it
 // LDS kept for the point lists of a tile
 constexpr size_t RES_PTS_LDS = 2048;
 
@@ -69,6 +74,7 @@ struct Group {
     Tile tv, ts;
     int off_v = 0, nblk_v = 0, off_s = 0, nblk_s = 0;
     int nfull_v = 0, nfull_s = 0;  // full-tile blocks at the head of each table
+    long end = 0;                  // engine clock of its last step
 };
 
 
@@ -339,35 +345,75 @@ int begin_shot(dn_ctx *c, int phase)
     return DN_OK;
 }
 
+// Planes that both sweeps of a step read or write, per cell
+int state_planes(const dn_ctx *c) { return 10 + (c->p.L ? 3 * c->p.L + 3 : 0); }
+
+// The shots of a group (indices into jobs) that go through a run of steps
+// together.  Up to 55e6 plane cells (220 MB) one part is the fastest; more
+// are packed into parts of 50e6 (200 MB; the last-level cache has 256 MB).
+// Elastic FDORDER 8: 3.7e6 cells 53 us a step, 5.0e6 70, 6.2e6 108, 7.8e6 133
+// in one part, where a part within the cache takes 14 us and 10 us per million
+// cells; three 4000x1200 grids 270 us a step in one part, 177 in three.
+std::vector<std::vector<int>> parts_of(const dn_engine *e, std::vector<int> v)
+{
+    constexpr long ONE = 55000000, PART = 50000000;
+    auto weight = [&](int k) {
+        const dn_ctx *c = e->jobs[k].ctx;
+        return (long)c->p.nx * c->p.ny * state_planes(c);
+    };
+    long all = 0;
+    for (int k : v) all += weight(k);
+    if (all <= ONE) return {v};
+    std::stable_sort(v.begin(), v.end(), [&](int a, int b) { return weight(a) > weight(b); });
+    std::vector<std::vector<int>> parts;
+    std::vector<long> load;
+    for (int k : v) {
+        size_t s = 0;
+        while (s < parts.size() && load[s] + weight(k) > PART) ++s;
+        if (s == parts.size()) {
+            parts.emplace_back();
+            load.push_back(0);
+        }
+        load[s] += weight(k);
+        parts[s].push_back(k);
+    }
+    return parts;
+}
+
 // group the running shots (resident: those no round carries) and upload the
 // launch tables of the sweeps
 int rebuild(dn_engine *e, bool resident)
 {
     HIP_OK(hipStreamSynchronize(e->stream));
     e->drop_graph();
-    std::map<std::tuple<int, int, int, int, int, int, int, int, int, int, int>, std::vector<int>> by;
+    typedef std::tuple<int, int, int, int, int, int, int, int, int, int, int> Key;
+    std::map<Key, std::vector<int>> alike;
     for (int k = 0; k < (int)e->jobs.size(); ++k) {
         if (resident && e->jobs[k].round >= 0) continue;
         const dn_ctx *c = e->jobs[k].ctx;
         const Tile &v = c->tile_v, &s = c->tile_s;
-        by[std::make_tuple(c->fdoh, c->p.L, e->jobs[k].phase, v.tbx, v.by, v.ty, v.vw, s.tbx, s.by, s.ty, s.vw)]
+        alike[std::make_tuple(c->fdoh, c->p.L, e->jobs[k].phase, v.tbx, v.by, v.ty, v.vw, s.tbx, s.by, s.ty, s.vw)]
             .push_back(k);
     }
+    std::vector<std::vector<int>> by;
+    for (const auto &kv : alike)
+        for (auto &part : parts_of(e, kv.second)) by.push_back(part);
     std::vector<BatchShot> shots;
     std::vector<BatchBlock> blk;
     e->groups.clear();
-    for (auto &kv : by) {
+    for (const auto &part : by) {
         Group g;
-        const dn_ctx *c0 = e->jobs[kv.second[0]].ctx;
+        const dn_ctx *c0 = e->jobs[part[0]].ctx;
         g.fdoh = c0->fdoh;
         g.L = c0->p.L;
-        g.sw = e->jobs[kv.second[0]].phase;
+        g.sw = e->jobs[part[0]].phase;
         g.tv = c0->tile_v;
         g.ts = c0->tile_s;
         std::vector<BatchBlock> bv, bs, lv, ls;  // full and lean blocks of each sweep
-        for (int k : kv.second) {
+        for (int k : part) {
             const Job &j = e->jobs[k];
             dn_ctx *c = j.ctx;
+            g.end = std::max(g.end, j.base + c->p.nt);
             BatchShot b{};
             b.a = c->a;
             const StepCtl base = j.phase == 0 ? base_ctl(c, 0, 1) : base_ctl(c, 2, 3);
@@ -428,26 +474,25 @@ int rebuild(dn_engine *e, bool resident)
     return DN_OK;
 }
 
-// step k of a run of steps
-void enqueue_step(dn_engine *e, int k)
+// a run of n steps from the clock's value `from`, then the clock moves on by
+// n; a group whose shots end before needs no more launches (from < 0: a run
+// that is captured once for any clock)
+void enqueue_run(dn_engine *e, int n, long from)
 {
-    for (const Group &g : e->groups)
-        launch_batch_vel(e->d_shots, e->d_blk + g.off_v, g.nblk_v, g.nfull_v, e->d_clock, k, g.tv, g.fdoh, g.sw, e->stream);
-    for (const Group &g : e->groups)
-        launch_batch_str(e->d_shots, e->d_blk + g.off_s, g.nblk_s, g.nfull_s, e->d_clock, k, g.ts, g.fdoh, g.L, e->stream);
-}
-
-// a run of n steps, then the clock moves on by n
-void enqueue_run(dn_engine *e, int n)
-{
-    for (int k = 0; k < n; ++k) enqueue_step(e, k);
+    for (const Group &g : e->groups) {
+        const int steps = from < 0 ? n : (int)std::min<long>(n, g.end - from + 1);
+        for (int k = 0; k < steps; ++k) {
+            launch_batch_vel(e->d_shots, e->d_blk + g.off_v, g.nblk_v, g.nfull_v, e->d_clock, k, g.tv, g.fdoh, g.sw, e->stream);
+            launch_batch_str(e->d_shots, e->d_blk + g.off_s, g.nblk_s, g.nfull_s, e->d_clock, k, g.ts, g.fdoh, g.L, e->stream);
+        }
+    }
     launch_batch_clock(e->d_clock, n, e->stream);
 }
 
 int capture(dn_engine *e)
 {
     HIP_OK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeRelaxed));
-    enqueue_run(e, e->graph_steps);
+    enqueue_run(e, e->graph_steps, -1);
     hipGraph_t g = nullptr;
     HIP_OK(hipStreamEndCapture(e->stream, &g));
     e->graph = g;
@@ -593,7 +638,7 @@ int dn_engine_launch(dn_engine *e, int nsteps)
         if (!e->gexec && (rc = capture(e))) return rc;
         for (; left >= e->graph_steps; left -= e->graph_steps) HIP_OK(hipGraphLaunch(e->gexec, e->stream));
     }
-    if (left > 0) enqueue_run(e, left);
+    if (left > 0) enqueue_run(e, left, e->clock - left);
     HIP_OK(hipGetLastError());
     return DN_OK;
 }

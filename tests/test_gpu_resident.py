@@ -243,3 +243,28 @@ def test_engine_gradient_rounds_equal_sweeps():
             ref.assemble()
             for w in range(6):
                 np.testing.assert_array_equal(g.gradient(w), ref.gradient(w), err_msg=f"{case[0].nx} gradient {w}")
+
+
+def test_engine_parts_equal_single_shots():
+    """Three grids that together exceed the last-level cache: the engine runs
+    them in parts, each through a whole run of steps, with and without a
+    graph, while a small shot ends between them."""
+    cases = [make_case(nx=nx, ny=ny, nt=nt, fdorder=8, fw=10, seismo=1, homogeneous=True, nrec=nx // 9, seed=k + 1)
+             for k, (nx, ny, nt) in enumerate([(2600, 900, 26), (2400, 1000, 37), (2500, 950, 30), (60, 50, 21)])]
+    print("parts of the engine's sweeps", flush=True)
+    shots = [context(c, True) for c in cases]
+    for g in shots:
+        g.forward()
+    want = [(g.seismogram(0), g.field(dnhip.F_SXX)) for g in shots]
+    for graph in (0, 8):
+        eng = dnhip.Engine()
+        eng.set_graph(graph)
+        for g in shots:
+            eng.attach(g)
+        while eng.step(16) > 0:
+            pass
+        for g, (s, f) in zip(shots, want):
+            assert eng.status(g) == 0
+            assert np.abs(f).max() > 0
+            np.testing.assert_array_equal(g.seismogram(0), s)
+            np.testing.assert_array_equal(g.field(dnhip.F_SXX), f)
