@@ -862,6 +862,28 @@ static int set_model_sh(dn_ctx *c, const float *vs, const float *rho, const floa
     return DN_OK;
 }
 
+// Elastic P/SV material on the device: the model arrays go up as they are
+// (rip and rjp hold them x-major for the moment) and become row-major planes
+// -- vp, vs, rho where the context keeps them, else g, f and muipjp, which
+// the averages then replace cell by cell.
+static int set_model_elastic(dn_ctx *c, const float *vp, const float *vs, const float *rho)
+{
+    const size_t n = (size_t)c->p.nx * c->p.ny, org = c->lay.origin();
+    const float *from[3] = {vp, vs, rho};
+    float *to[3] = {c->vp ? c->vp : c->g, c->vp ? c->vs : c->f, c->vp ? c->rho : c->muipjp};
+    int rc;
+    for (int k = 0; k < 3; ++k) {
+        float *stage = k == 1 ? c->rjp : c->rip;
+        if ((rc = upload(c, stage, from[k], n))) return rc;
+        launch_transpose(stage, to[k], c->lay, c->stream);
+    }
+    const MaterialPlanes m{to[0] + org, to[1] + org, to[2] + org, c->rip + org, c->rjp + org, c->muipjp + org,
+                           c->f + org,  c->g + org};
+    launch_material(m, c->lay, c->p.invmat1, c->stream);
+    HIP_OK(hipGetLastError());
+    return DN_OK;
+}
+
 int dn_set_model(dn_ctx *c, const float *vp, const float *vs, const float *rho, const float *taus,
                  const float *taup)
 {
@@ -874,22 +896,15 @@ int dn_set_model(dn_ctx *c, const float *vp, const float *vs, const float *rho, 
     std::string err;
     int rc = check_stability(c->p, c->setup.hc, vp, vs, rho, taus, taup, err);
     if (rc) return fail(rc, err);
-    prepare_material(c->p, c->lay, vp, vs, rho, taus, taup, c->mat);
     const size_t pl = c->lay.plane();
-    if ((rc = upload(c, c->rip, c->mat.rip.data(), pl)) || (rc = upload(c, c->rjp, c->mat.rjp.data(), pl)))
-        return rc;
     if (c->p.L == 0) {
-        if ((rc = upload(c, c->muipjp, c->mat.muipjp.data(), pl)) || (rc = upload(c, c->f, c->mat.f.data(), pl)) ||
-            (rc = upload(c, c->g, c->mat.g.data(), pl)))
-            return rc;
-    }
-    if (c->vp) {
-        if ((rc = upload(c, c->vp, c->mat.vp.data(), pl)) || (rc = upload(c, c->vs, c->mat.vs.data(), pl)) ||
-            (rc = upload(c, c->rho, c->mat.rho.data(), pl)))
-            return rc;
-    }
-    if (c->p.L > 0) {
-        if ((rc = upload(c, c->vmu, c->mat.vmu.data(), pl)) || (rc = upload(c, c->vts, c->mat.vts.data(), pl)) ||
+        if ((rc = set_model_elastic(c, vp, vs, rho))) return rc;
+    } else {
+        prepare_material(c->p, c->lay, vp, vs, rho, taus, taup, c->mat);
+        if ((rc = upload(c, c->rip, c->mat.rip.data(), pl)) || (rc = upload(c, c->rjp, c->mat.rjp.data(), pl)) ||
+            (c->vp && ((rc = upload(c, c->vp, c->mat.vp.data(), pl)) || (rc = upload(c, c->vs, c->mat.vs.data(), pl)) ||
+                       (rc = upload(c, c->rho, c->mat.rho.data(), pl)))) ||
+            (rc = upload(c, c->vmu, c->mat.vmu.data(), pl)) || (rc = upload(c, c->vts, c->mat.vts.data(), pl)) ||
             (rc = upload(c, c->vpi, c->mat.vpi.data(), pl)) || (rc = upload(c, c->vtp, c->mat.vtp.data(), pl)) ||
             (rc = upload(c, c->vmuij, c->mat.vmuij.data(), pl)) || (rc = upload(c, c->vtsij, c->mat.vtsij.data(), pl)) ||
             (rc = upload(c, c->fs_fjm, c->mat.fs_fjm.data(), c->p.nx + 1)) ||
@@ -919,9 +934,6 @@ int dn_set_model(dn_ctx *c, const float *vp, const float *vs, const float *rho, 
     // host staging of the device-layout material is no longer needed
     c->mat.rip.clear(); c->mat.rip.shrink_to_fit();
     c->mat.rjp.clear(); c->mat.rjp.shrink_to_fit();
-    c->mat.muipjp.clear(); c->mat.muipjp.shrink_to_fit();
-    c->mat.f.clear(); c->mat.f.shrink_to_fit();
-    c->mat.g.clear(); c->mat.g.shrink_to_fit();
     c->mat.vp.clear(); c->mat.vp.shrink_to_fit();
     c->mat.vs.clear(); c->mat.vs.shrink_to_fit();
     c->mat.rho.clear(); c->mat.rho.shrink_to_fit();

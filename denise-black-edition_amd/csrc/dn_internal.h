@@ -50,7 +50,6 @@ struct HostSetup {
 // Material fields prepared on the host in the device layout.
 struct HostMaterial {
     std::vector<float> rip, rjp;           // 1/rho at i+1/2 and j+1/2
-    std::vector<float> muipjp, f, g;       // elastic: uipjp, rho vs^2, rho(vp^2-2vs^2)
     // viscoelastic: relaxed moduli and relaxation times; the update rebuilds
     // fipjp, f, g (with DT) and the per-mechanism d, e, dip from them
     std::vector<float> vmu, vts, vpi, vtp, vmuij, vtsij;
@@ -289,6 +288,13 @@ void launch_energy(const KArgs &a, float *W, void *stream);
 void launch_store(const KArgs &a, float *const fwd[5], long k, void *stream);
 void launch_assemble(const KArgs &a, const float *wc, const float *wcu, const float *wcr, float *gvp,
                      float *gvs, float *grho, int invmat1, int physics, void *stream);
+// model planes of an elastic P/SV context (dn_material of dn_kernels.hip)
+struct MaterialPlanes {
+    const float *vp, *vs, *rho;  // first cells; mode 0: g, f and muipjp themselves
+    float *rip, *rjp, *muipjp, *f, *g;
+};
+void launch_transpose(const float *xmajor, float *plane, const Layout &lay, void *stream);
+void launch_material(const MaterialPlanes &m, const Layout &lay, int invmat1, void *stream);
 void launch_residual(const DevAcq &q, int comp, const float *obs, float dt, float w, void *stream);
 void launch_l2(const DevAcq &q, int comp, void *stream);
 int l2_scratch_doubles();  // doubles behind DevAcq::l2

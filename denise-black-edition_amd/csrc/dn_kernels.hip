@@ -240,6 +240,71 @@ __global__ __launch_bounds__(256) void k_l2_sum(DevAcq q)
     if (threadIdx.x == 0) q.l2[0] = q.l2[0] + tot;
 }
 
+// Model planes of an elastic P/SV context (dn_set_model): a memory-bound
+// pass, 1 plane in and out per array for the transposition, 3 + 4 and 1 + 1
+// planes for the averages.  On the host the same took most of a gradient
+// evaluation's set-up: 2000x600 21.6 ms per model, now 1.4, nearly all of it
+// the upload of three arrays, the host's copy and the stability check.
+//
+// x-major (i, j) -> row-major plane (j, i) through a tile in LDS
+__global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ in, float *__restrict__ out, int nx, int ny,
+                                                   int pitch)
+{
+    __shared__ float t[32][33];
+    const int i0 = blockIdx.x * 32, j0 = blockIdx.y * 32;
+    for (int k = threadIdx.y; k < 32; k += 8) {
+        const int i = i0 + k, j = j0 + threadIdx.x;
+        if (i < nx && j < ny) t[k][threadIdx.x] = in[(long)i * ny + j];
+    }
+    __syncthreads();
+    for (int k = threadIdx.y; k < 32; k += 8) {
+        const int j = j0 + k, i = i0 + threadIdx.x;
+        if (i < nx && j < ny) out[(long)j * pitch + i] = t[threadIdx.x][k];
+    }
+}
+
+// Reciprocal arithmetic-mean densities at (i+1/2, j) and (i, j+1/2)
+// (src/av_rho.c:5-28; the neighbours of the last row and column are the first
+// ones) and the moduli f, g.  rip and rjp held x-major arrays, so their
+// padding is written too; f and g may be the planes of vs and vp (same cell).
+__global__ __launch_bounds__(256) void k_density_moduli(MaterialPlanes m, Layout lay, int invmat1)
+{
+    const int col = blockIdx.y * 256 + threadIdx.x, row = blockIdx.x;
+    if (col >= lay.pitch) return;
+    const int i = col - HX, j = row - HY;
+    const long o = (long)j * lay.pitch + i;
+    float ri = 0.0f, rj = 0.0f;
+    if (i >= 0 && i < lay.nx && j >= 0 && j < lay.ny) {
+        const float r = m.rho[o];
+        const float rx = m.rho[(long)j * lay.pitch + (i + 1 < lay.nx ? i + 1 : 0)];
+        const float ry = m.rho[(long)(j + 1 < lay.ny ? j + 1 : 0) * lay.pitch + i];
+        rj = (float)(1.0 / (0.5 * (r + ry)));
+        ri = (float)(1.0 / (0.5 * (r + rx)));
+        if (r < 1e-4 && ry < 1e-4) rj = 0.0f;
+        if (r < 1e-4 && rx < 1e-4) ri = 0.0f;
+        const float p = m.vp[o], u = m.vs[o];
+        m.f[o] = invmat1 == 3 ? u : r * u * u;
+        m.g[o] = invmat1 == 3 ? p : r * ((p * p) - 2 * u * u);
+    }
+    m.rip[o] = ri;
+    m.rjp[o] = rj;
+}
+
+// harmonic average of the shear modulus over the four cells around
+// (i+1/2, j+1/2) (src/av_mue.c:5-51)
+__global__ __launch_bounds__(256) void k_shear(const float *__restrict__ mu, float *__restrict__ out, int nx, int ny,
+                                               int pitch)
+{
+    const int i = blockIdx.y * 256 + threadIdx.x, j = blockIdx.x;
+    if (i >= nx) return;
+    const int ix = i + 1 < nx ? i + 1 : 0, jy = j + 1 < ny ? j + 1 : 0;
+    const float u1 = mu[(long)j * pitch + i], u2 = mu[(long)j * pitch + ix];
+    const float u3 = mu[(long)jy * pitch + i], u4 = mu[(long)jy * pitch + ix];
+    float v = (float)(4.0 / ((1.0 / u1) + (1.0 / u2) + (1.0 / u3) + (1.0 / u4)));
+    if (u1 == 0.0f || u2 == 0.0f || u3 == 0.0f || u4 == 0.0f) v = 0.0f;
+    out[(long)j * pitch + i] = v;
+}
+
 }  // namespace
 
 // Tile shapes compiled into the library: X(TBX, BY, TY, name), each in its
@@ -338,6 +403,19 @@ void launch_assemble(const KArgs &a, const float *wc, const float *wcu, const fl
     dim3 g((unsigned)((n + 255) / 256));
     hipLaunchKernelGGL(k_assemble, g, dim3(256), 0, (hipStream_t)stream, a, wc, wcu, wcr, gvp, gvs, grho,
                        invmat1, physics);
+}
+
+void launch_transpose(const float *xmajor, float *plane, const Layout &lay, void *stream)
+{
+    hipLaunchKernelGGL(k_transpose, dim3((lay.nx + 31) / 32, (lay.ny + 31) / 32), dim3(32, 8), 0, (hipStream_t)stream,
+                       xmajor, plane + lay.origin(), lay.nx, lay.ny, lay.pitch);
+}
+
+void launch_material(const MaterialPlanes &m, const Layout &lay, int invmat1, void *stream)
+{
+    const dim3 all(lay.rows, (lay.pitch + 255) / 256), cells(lay.ny, (lay.nx + 255) / 256);
+    hipLaunchKernelGGL(k_density_moduli, all, dim3(256), 0, (hipStream_t)stream, m, lay, invmat1);
+    hipLaunchKernelGGL(k_shear, cells, dim3(256), 0, (hipStream_t)stream, m.f, m.muipjp, lay.nx, lay.ny, lay.pitch);
 }
 
 void launch_residual(const DevAcq &q, int comp, const float *obs, float dt, float w, void *stream)

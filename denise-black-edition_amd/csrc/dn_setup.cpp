@@ -170,10 +170,27 @@ int check_stability(const dn_params &p, const float hc[7], const float *vp, cons
 {
     const size_t n = (size_t)p.nx * p.ny;
     float cmax_s = 0.0f, cmax_p = 0.0f;
-    if (p.L == 0) {
+    if (p.L == 0 && p.invmat1 != 3) {
+        // several maxima side by side: one alone waits for itself
+        float ms[8] = {}, mp[8] = {};
+        size_t k = 0;
+        for (; k + 8 <= n; k += 8)
+            for (int q = 0; q < 8; ++q) {
+                ms[q] = ms[q] < vs[k + q] ? vs[k + q] : ms[q];
+                mp[q] = mp[q] < vp[k + q] ? vp[k + q] : mp[q];
+            }
+        for (; k < n; ++k) {
+            ms[0] = ms[0] < vs[k] ? vs[k] : ms[0];
+            mp[0] = mp[0] < vp[k] ? vp[k] : mp[0];
+        }
+        for (int q = 0; q < 8; ++q) {
+            cmax_s = cmax_s < ms[q] ? ms[q] : cmax_s;
+            cmax_p = cmax_p < mp[q] ? mp[q] : cmax_p;
+        }
+    } else if (p.L == 0) {
         for (size_t k = 0; k < n; ++k) {
-            float cs = p.invmat1 == 3 ? (float)std::sqrt(vs[k] / rho[k]) : vs[k];
-            float cp = p.invmat1 == 3 ? (float)std::sqrt((vp[k] + 2.0 * vs[k]) / rho[k]) : vp[k];
+            float cs = (float)std::sqrt(vs[k] / rho[k]);
+            float cp = (float)std::sqrt((vp[k] + 2.0 * vs[k]) / rho[k]);
             if (cmax_s < cs) cmax_s = cs;
             if (cmax_p < cp) cmax_p = cp;
         }
@@ -252,7 +269,8 @@ struct Ring {
 
 }  // namespace
 
-// Material averaging and coefficient preparation:
+// Viscoelastic material averaging and coefficient preparation (elastic
+// material is prepared on the device, dn_kernels.hip):
 // src/av_mue.c:5-51, src/av_rho.c:5-28, src/av_tau.c:5-15,
 // src/PSV/prepare_update_s_visc_PSV.c:8-94 (peta: src/PSV/readmod_visc_PSV.c:29-32),
 // per-column free-surface coefficients of src/PSV/surface_visc_PML_PSV.c:36-169.
@@ -269,9 +287,6 @@ void prepare_material(const dn_params &p, const Layout &lay, const float *vp, co
     auto dev = [&](int j, int i) { return lay.origin() + (size_t)lay.off(j, i); };
     m.rip.assign(plane, 0.0f);
     m.rjp.assign(plane, 0.0f);
-    m.muipjp.assign(plane, 0.0f);
-    m.f.assign(plane, 0.0f);
-    m.g.assign(plane, 0.0f);
     m.vp.assign(plane, 0.0f);
     m.vs.assign(plane, 0.0f);
     m.rho.assign(plane, 0.0f);
@@ -302,18 +317,7 @@ void prepare_material(const dn_params &p, const Layout &lay, const float *vp, co
             if (R.at(j, i) < 1e-4 && R.at(j, i + 1) < 1e-4) ri = 0.0f;
             m.rjp[o] = rj;
             m.rip[o] = ri;
-            if (L == 0) {
-                m.muipjp[o] = mu_h;
-                if (p.invmat1 == 3) {
-                    m.f[o] = U.at(j, i);
-                    m.g[o] = PI.at(j, i);
-                } else {
-                    m.f[o] = R.at(j, i) * U.at(j, i) * U.at(j, i);
-                    m.g[o] = R.at(j, i) * ((PI.at(j, i) * PI.at(j, i)) - 2 * U.at(j, i) * U.at(j, i));
-                }
-            }
         }
-    if (L == 0) return;
 
     Ring TS(NX, NY), TP(NX, NY);
     TS.load(taus);
