@@ -1,5 +1,5 @@
-"""Set-up work of a shot on the device against its host definition: the model
-planes of an elastic P/SV context."""
+"""Work around a shot's time loop on the device against its host definition:
+the model planes of an elastic P/SV context, the residuals of its traces."""
 import numpy as np
 import pytest
 
@@ -47,3 +47,39 @@ def test_elastic_model_planes(nx, ny, invmat1, mode):
     for k in range(4):
         assert np.abs(o.seismogram(k)).max() > 0
         np.testing.assert_array_equal(g.seismogram(k), o.seismogram(k))
+
+
+@pytest.mark.parametrize("nt", [2, 255, 256, 257, 530])
+@pytest.mark.parametrize("ntr", [1, 15, 16, 17, 50])
+def test_residual_traces(ntr, nt):
+    """Edges of the 16-trace, 256-sample pieces: the time integral is one
+    float32 chain per trace, so every sample is the host chain's."""
+    case = make_case(nx=120, ny=40, nt=nt, fw=5, seismo=1, mode=1, nrec=ntr)
+    p, m, src, sig, rec = case
+    g = dnhip.Context(p)
+    g.set_model(m["vp"], m["vs"], m["rho"])
+    g.set_sources(src, sig)
+    g.set_receivers(rec)
+    g.forward()
+    rng = np.random.default_rng(nt + ntr)
+    obs = [rng.standard_normal((ntr, nt)).astype(np.float32) for _ in range(2)]
+    print(f"residuals of {ntr} traces, {nt} samples", flush=True)
+    for w in (1.0, 0.3):
+        g.set_residual_weights(w, 1.0)
+        l2 = g.residuals(obs[0], obs[1], None, 1)
+        want = 0.0
+        for k in range(2):
+            f = np.float32(w if k == 0 else 1.0)
+            s = g.seismogram(k).reshape(ntr, nt) * f
+            d = obs[k] * f
+            d[:, 0] = s[:, 0]
+            x = np.float32(p.dt) * (s - d)
+            r = np.zeros_like(x)
+            acc = np.zeros(ntr, np.float32)
+            for n in range(nt):
+                acc = acc + x[:, n]
+                r[:, nt - 1 - n] = acc
+            np.testing.assert_array_equal(g.adjoint_sources(k).reshape(ntr, nt), r)
+            want += float((0.5 * r.astype(np.float64) ** 2).sum())
+        # a sum of n positive terms in any order: n roundings at most
+        assert abs(l2 - want) <= 2 * ntr * nt * 2.3e-16 * want
