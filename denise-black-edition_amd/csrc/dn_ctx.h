@@ -156,6 +156,15 @@ struct dn_ctx {
         *ptr = nullptr;
         return dalloc(ptr, nbytes);
     }
+    // a buffer of nbytes: the one there if it has that size
+    int resize(void **ptr, size_t nbytes)
+    {
+        for (auto &pr : allocs)
+            if (*ptr && pr.first == *ptr && pr.second == (nbytes ? nbytes : 4)) return DN_OK;
+        if (*ptr) dfree(*ptr);
+        *ptr = nullptr;
+        return dalloc(ptr, nbytes);
+    }
     ~dn_ctx()
     {
         if (device >= 0) (void)hipSetDevice(device);
