@@ -408,17 +408,17 @@ int validate(const dn_params *p)
 
 int dn::zero_state(dn_ctx *c)
 {
-    const size_t pb = c->lay.plane() * sizeof(float);
+    ZeroList z;
+    const size_t pl = c->lay.plane();
     for (int k = 0; k < F_N; ++k)
-        if (c->fld[k]) HIP_OK(hipMemsetAsync(c->fld[k], 0, pb, c->stream));
-    if (c->p.L > 0) {
-        HIP_OK(hipMemsetAsync(c->rmem, 0, pb * c->p.L, c->stream));
-        HIP_OK(hipMemsetAsync(c->pmem, 0, pb * c->p.L, c->stream));
-        HIP_OK(hipMemsetAsync(c->qmem, 0, pb * c->p.L, c->stream));
-    }
+        if (c->fld[k]) z.add(c->fld[k], pl);
+    if (c->p.L > 0)
+        for (float *m : {c->rmem, c->pmem, c->qmem}) z.add(m, pl * c->p.L);
     const size_t nxb = (size_t)c->p.ny * 2 * c->p.fw, nyb = (size_t)2 * c->p.fw * c->p.nx;
-    for (int k = 0; k < 9; ++k) HIP_OK(hipMemsetAsync(c->psi[k], 0, (k < 5 ? nxb : nyb) * sizeof(float) + 4, c->stream));
-    HIP_OK(hipMemsetAsync(c->acq.nan_step, 0, 2 * sizeof(int), c->stream));
+    for (int k = 0; k < 9; ++k) z.add(c->psi[k], (k < 5 ? nxb : nyb) + 1);
+    z.add(c->acq.nan_step, 2);
+    launch_zero(z, c->stream);
+    HIP_OK(hipGetLastError());
     return DN_OK;
 }
 

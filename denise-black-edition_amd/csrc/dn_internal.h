@@ -293,6 +293,22 @@ struct MaterialPlanes {
     const float *vp, *vs, *rho;  // first cells; mode 0: g, f and muipjp themselves
     float *rip, *rjp, *muipjp, *f, *g;
 };
+// buffers that one launch clears, in 4-byte words
+struct ZeroList {
+    static constexpr int MAX = 32;
+    void *ptr[MAX];
+    size_t end[MAX];  // 16-byte pieces up to and with this buffer
+    size_t words[MAX];
+    int n = 0;
+    void add(void *p, size_t w)
+    {
+        ptr[n] = p;
+        words[n] = w;
+        end[n] = (n ? end[n - 1] : 0) + (w + 3) / 4;
+        ++n;
+    }
+};
+void launch_zero(const ZeroList &z, void *stream);
 void launch_transpose(const float *xmajor, float *plane, const Layout &lay, void *stream);
 void launch_material(const MaterialPlanes &m, const Layout &lay, int invmat1, void *stream);
 void launch_residual(const DevAcq &q, int comp, const float *obs, float dt, float w, void *stream);

@@ -255,6 +255,25 @@ __global__ __launch_bounds__(256) void k_l2_sum(DevAcq q)
     if (threadIdx.x == 0) q.l2[0] = q.l2[0] + tot;
 }
 
+// Clears the state of a shot, twenty buffers, in one launch: a memset each
+// cost 2 us and more of launches (120x80: 58 us of a 1.2 ms run).
+__global__ __launch_bounds__(256) void k_zero(ZeroList z)
+{
+    typedef unsigned U4 __attribute__((ext_vector_type(4)));
+    const size_t all = z.end[z.n - 1], step = (size_t)gridDim.x * 256;
+    int b = 0;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < all; i += step) {
+        while (i >= z.end[b]) ++b;
+        const size_t k = 4 * (i - (b ? z.end[b - 1] : 0)), w = z.words[b];
+        unsigned *p = (unsigned *)z.ptr[b] + k;
+        if (k + 4 <= w) {
+            *reinterpret_cast<U4 *>(p) = (U4)(0u);
+        } else {
+            for (size_t e = 0; e < w - k; ++e) p[e] = 0u;
+        }
+    }
+}
+
 // Model planes of an elastic P/SV context (dn_set_model): a memory-bound
 // pass, 1 plane in and out per array for the transposition, 3 + 4 and 1 + 1
 // planes for the averages.  On the host the same took most of a gradient
@@ -418,6 +437,13 @@ void launch_assemble(const KArgs &a, const float *wc, const float *wcu, const fl
     dim3 g((unsigned)((n + 255) / 256));
     hipLaunchKernelGGL(k_assemble, g, dim3(256), 0, (hipStream_t)stream, a, wc, wcu, wcr, gvp, gvs, grho,
                        invmat1, physics);
+}
+
+void launch_zero(const ZeroList &z, void *stream)
+{
+    if (z.n == 0) return;
+    const size_t blocks = (z.end[z.n - 1] + 1023) / 1024;
+    hipLaunchKernelGGL(k_zero, dim3((unsigned)std::min<size_t>(blocks, 1u << 20)), dim3(256), 0, (hipStream_t)stream, z);
 }
 
 void launch_transpose(const float *xmajor, float *plane, const Layout &lay, void *stream)

@@ -83,3 +83,28 @@ def test_residual_traces(ntr, nt):
             want += float((0.5 * r.astype(np.float64) ** 2).sum())
         # a sum of n positive terms in any order: n roundings at most
         assert abs(l2 - want) <= 2 * ntr * nt * 2.3e-16 * want
+
+
+@pytest.mark.parametrize("nx,ny,L", [(29, 21, 0), (130, 67, 3)])
+def test_state_is_cleared(nx, ny, L):
+    """A second run of a context starts from zeros in every field, memory
+    variable and CPML array (odd lengths among them)."""
+    case = make_case(nx=nx, ny=ny, nt=40, L=L, fw=5, seismo=4, homogeneous=True)
+    p, m, src, sig, rec = case
+    g = dnhip.Context(p)
+    g.set_model(m["vp"], m["vs"], m["rho"], m["taus"], m["taup"])
+    g.set_sources(src, sig)
+    g.set_receivers(rec)
+    print(f"cleared state {nx}x{ny} L {L}", flush=True)
+    out = []
+    for _ in range(2):
+        g.forward()
+        out.append([g.field(k) for k in range(7)] + [g.psi(k) for k in range(9)] +
+                   [g.memvar(w, l + 1) for w in range(3) for l in range(L)])
+    assert np.abs(out[0][0]).max() > 0
+    for x, y in zip(*out):
+        np.testing.assert_array_equal(x, y)
+    g.set_sources(src, 0.0 * sig)
+    g.forward()
+    assert all(not np.any(g.field(k)) for k in range(7)) and all(not np.any(g.psi(k)) for k in range(9))
+    assert all(not np.any(g.memvar(w, l + 1)) for w in range(3) for l in range(L))
