@@ -484,7 +484,7 @@ size_t dn::res_lds(const ResPlan &pl, const ResPoints &pt, int sw)
 // sweep shape or cache policy chosen by the caller.
 bool dn::res_applies(const dn_ctx *c, int sw)
 {
-    if (!c->res.ok || c->sweeps_chosen || !res_compiled(c->a.physics, c->p.L, sw)) return false;
+    if (!c->res.ok || c->sweeps_chosen) return false;
     if (!c->res_pts.ok[2 * sw] || !c->res_pts.ok[2 * sw + 1]) return false;
     if (c->p.L > 0 && !c->tau_const) return false;  // relaxation times as planes
     // the curl at acoustic receivers differences vx along y and vy along x,
@@ -499,10 +499,10 @@ bool dn::res_applies(const dn_ctx *c, int sw)
     return c->p.dh >= 0x1p-60f && c->p.dh <= 0x1p60f;
 }
 
-// the point lists of a plan fit beside its fields
+// a kernel is compiled for the plan, and its point lists fit beside its fields
 bool dn::res_points_fit(const dn_ctx *c, const ResPlan &pl, const ResPoints &pt, int sw)
 {
-    return pt.most[2 * sw] <= RES_ENT && pt.most[2 * sw + 1] <= RES_ENT &&
+    return res_compiled(c->a.physics, c->p.L, sw, pl.ry) && pt.most[2 * sw] <= RES_ENT && pt.most[2 * sw + 1] <= RES_ENT &&
            res_lds(pl, pt, sw) <= res_pool_lds(c->res_pool);
 }
 

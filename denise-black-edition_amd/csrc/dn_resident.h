@@ -49,8 +49,8 @@ struct ResKernel {
     const ResBlock *blk;
 };
 
-// is there a compiled kernel for this run (sw 0 forward, 1 adjoint)
-bool res_compiled(int physics, int L, int sw);
+// is there a compiled kernel for this run (sw 0 forward, 1 adjoint) with ry rows per thread
+bool res_compiled(int physics, int L, int sw, int ry);
 // enqueue one launch of as many workgroups, with the threads, LDS and thread
 // shape of pl; false when the runtime refuses it
 bool res_launch(const ResKernel &k, const ResPlan &pl, int blocks, int fdoh, int sw, void *stream);

@@ -22,11 +22,14 @@ constexpr int res_maxt(int ry, int vx, int F, int L)
 {
     return ry > 1 ? 512 : vx == 1 ? 1024 : vx == 2 ? (F <= 4 ? 1024 : 768) : (F <= 4 && L == 0 ? 768 : 512);
 }
-// Rows per thread, at most.  Three relaxation mechanisms (nine memory
-// variables per cell) spill with several rows: 1500x400 forward 23.7 us a
-// step against the sweeps' 22.4, adjoint 30.6 against 28.9.  With two
-// mechanisms 2000x600 takes 27.4 against 30.8 us, 1500x400 16.2 against 20.3.
-constexpr int res_rows(int L) { return L < 3 ? 3 : 1; }
+// Rows per thread, at most (sw: 0 forward, 1 adjoint).  Three relaxation
+// mechanisms (nine memory variables per cell) spill with several rows: the
+// sweeps were as fast or faster.  So do viscoelastic adjoint runs, and a trial
+// build of one with three mechanisms and two rows ended in a memory fault of
+// unknown cause: they take one-row shapes or the sweeps.  Two mechanisms,
+// forward: 2000x600 27 us a step against 31 in the sweeps, 1500x400 16
+// against 20.
+constexpr int res_rows(int L, int sw) { return L == 0 || (L < 3 && sw == 0) ? 3 : 1; }
 constexpr int res_width(int ry) { return ry == 1 ? 32 : ry == 2 ? 64 : 72; }
 constexpr int RES_ENT = 256;     // sources and receivers of one tile and sweep kept in LDS, at most
 constexpr int res_ki(int F) { return F <= 4 ? 4 : 6; }  // halo words per thread and exchange, at most
