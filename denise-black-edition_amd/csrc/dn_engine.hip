@@ -55,15 +55,15 @@ struct Round {
 };
 
 // Fewest steps of a run that the rounds carry: a launch loads and stores the
-// whole state of its shots.  Three 400x200 shots, runs of 8 steps: 14.7 us a
-// step (sweeps 25.5), 32 steps 8.7; one 2000x600 shot 24.7 (32.3) and 12.1.
+// whole state of its shots.  Three 400x200 shots, runs of 8 steps: 13.3 us a
+// step (sweeps 25.9), 32 steps 7.2; one 2000x600 shot 22.5 (32.4) and 10.3.
 constexpr int RES_MIN_STEPS = 8;
 // Shots in the sweeps beside a round: while the sweeps' shots stay within
 // the last-level cache (about 4.5e6 cells) a million cells more cost them 10
-// us a step, and the round 4.4 + 7.4 us; past it they need another 14 us.
-// 1.1e6 cells beside 1.9e6 in the sweeps: 48.9 us with the round, 47.7
-// without; 0.34e6: 42.5 and 38.8.  Beside 5.0e6: 1.1e6 81.4 and 96.1, 0.79e6
-// 79.7 and 89.7; beside 7.8e6: 1.1e6 119.5 and 119.5, 0.34e6 142.6 and 110.2.
+// us a step, and the round 3.5 + 6 us; past it they need another 14 us.
+// 1.1e6 cells beside 1.9e6 in the sweeps: 46.4 us with the round, 47.7
+// without, beside 3.7e6 63.6 and 70.8; 0.34e6 beside 1.9e6: 42.5 and 38.8.
+// Beside 5.0e6: 1.1e6 90.0 and 100.7, 0.79e6 88.6 and 92.9.
 constexpr long RES_LLC_CELLS = 4500000;
 constexpr long RES_MIN_CELLS[2] = {1100000, 700000};  // of a round, within the cache and past it
 // LDS kept for the point lists of a tile
@@ -149,8 +149,8 @@ int grow(T **p, size_t *cap, size_t n)
 }
 
 // Which shots the chip-resident loop carries, and the rounds it does so in.
-// A round takes about 4.4 us a step and 1.9 us per thousand cells of a tile
-// (FDORDER 8, elastic: 340 cells 5.0 us, 4690 cells 13.3), so the fewest win:
+// A round takes about 3.5 us a step and 1.5 us per thousand cells of a tile
+// (FDORDER 8, elastic: 340 cells 4.0 us, 4690 cells 10.6), so the fewest win:
 // shots are packed largest first by the fewest tiles that hold them, and the
 // CUs left over are then dealt out in proportion.
 int plan_rounds(dn_engine *e)

@@ -88,9 +88,10 @@ ResPlan res_plan(const dn_params &p, int ncu, size_t lds_max, int shape)
 {
     ResPlan best;
     // The fewest cells per thread that fit: more waves share a CU's four SIMDs
-    // and hide each other's latencies.  FDORDER 8 elastic steps: 500x174 5.1 us
-    // with 1 x 1 cells per thread, 6.3 with 1 x 2, 7.2 with 1 x 4, 10.0 with
-    // 2 x 4; 611x303 5.9 with 1 x 2, 7.6 with 1 x 4, 10.2 with 2 x 4.
+    // and hide each other's latencies.  FDORDER 8 elastic steps: 500x174 4.0 us
+    // with 1 x 1 cells per thread, 4.8 with 1 x 2, 6.3 with 1 x 4, 7.4 with
+    // 2 x 4, 9.3 with 3 x 4; 1000x400 6.3 with 1 x 2, 7.8 with 1 x 4, 7.7 with
+    // 2 x 4, 9.5 with 3 x 4; 1500x600 8.6 with 2 x 4, 10.3 with 3 x 4.
     for (int s = shape < 0 ? 0 : shape; s < (shape < 0 ? RES_SHAPES : shape + 1) && !best.ok; ++s) {
         Cut c(p, lds_max, s);
         double cost = 0.0;

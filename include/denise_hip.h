@@ -231,7 +231,9 @@ int dn_get_hc(dn_ctx *ctx, float *out7);
  * shapes (tbx,by,ty,vw): (64,4,1,1), (128,2,1,1), (256,1,1,1), (64,4,2,1),
  * (128,2,4,1), (64,8,2,1), (64,4,1,4), (64,4,2,4), (64,2,4,4), (64,4,1,2),
  * (128,2,2,2), (64,4,2,2); VTI/TTI stress sweeps take vw = 1 only.
- * Results do not depend on the shapes.  No reference
+ * Results do not depend on the shapes.  A context whose caller chose a shape
+ * runs the sweeps; others run in the chip-resident time loop where their grid
+ * fits it (up to about 1.3 million elastic cells).  No reference
  * counterpart: the reference has no GPU launch shapes. */
 int dn_set_tile(dn_ctx *ctx, int sweep, int tbx, int by, int ty, int vw);
 int dn_get_tile(dn_ctx *ctx, int sweep, int *tbx, int *by, int *ty, int *vw);
@@ -240,7 +242,8 @@ int dn_get_tile(dn_ctx *ctx, int sweep, int *tbx, int *by, int *ty, int *vw);
  * planes a step reads once (material and coefficient planes) and streaming
  * stores of the memory variables, so that they do not displace from the
  * caches the wavefields the next sweep reads.  sweep 0 velocity, 1 stress,
- * -1 both (set only).  Results do not depend on it.  No reference
+ * -1 both (set only).  Setting it selects the sweeps, as dn_set_tile does.
+ * Results do not depend on it.  No reference
  * counterpart. */
 int dn_set_store_hint(dn_ctx *ctx, int sweep, int streaming);
 int dn_get_store_hint(dn_ctx *ctx, int sweep, int *streaming);
