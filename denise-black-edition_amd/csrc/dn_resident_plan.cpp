@@ -71,8 +71,12 @@ struct Cut {
                     const int h = std::min(q.th, p.ny - by * q.th), LP = res_width(ry) + 2 * HP;
                     const int rows = nf * (h + 2 * F) - (nf == 5 ? 2 * F : 0);
                     const size_t prof = (size_t)(8 * (2 * p.fw + 1) + 3) / 4 * 4;
-                    const size_t psi = (size_t)2 * n * ((b.nx ? h * q.ncx * 4 : 0) + (b.ny ? q.ncy * q.tw : 0));
-                    q.lds = std::max(q.lds, ((size_t)rows * LP + prof + psi) * sizeof(float) + 16);
+                    const size_t psi_x = b.nx ? (size_t)2 * n * h * q.ncx * 4 : 0, psi_y = b.ny ? (size_t)2 * n * q.ncy * q.tw : 0;
+                    // threads whose last rows lie below the tile read them too, and
+                    // drop what they get: rows past the last plane, rows past the x memory
+                    const size_t below = (size_t)((h + ry - 1) / ry * ry - h), fields = (size_t)rows * LP;
+                    const size_t behind = prof + std::max(psi_x + psi_y, psi_x + (b.nx ? below * q.ncx * 4 : 0));
+                    q.lds = std::max(q.lds, (fields + std::max(behind, below * LP)) * sizeof(float) + 16);
                 }
             if (q.lds > lds_max) continue;
             q.ok = true;
