@@ -502,7 +502,7 @@ bool dn::res_applies(const dn_ctx *c, int sw)
 // a kernel is compiled for the plan, and its point lists fit beside its fields
 bool dn::res_points_fit(const dn_ctx *c, const ResPlan &pl, const ResPoints &pt, int sw)
 {
-    return res_compiled(c->a.physics, c->p.L, sw, pl.ry) && pt.most[2 * sw] <= RES_ENT && pt.most[2 * sw + 1] <= RES_ENT &&
+    return res_compiled(c->fdoh, c->a.physics, c->p.L, sw, pl.ry) && pt.most[2 * sw] <= RES_ENT && pt.most[2 * sw + 1] <= RES_ENT &&
            res_lds(pl, pt, sw) <= res_pool_lds(c->res_pool);
 }
 

@@ -171,7 +171,7 @@ int plan_rounds(dn_engine *e)
         if (!j.sweeps && res_applies(j.ctx, j.phase))
             for (int s = 0; s < RES_SHAPES; ++s) {
                 const ResPlan pl = res_least(j.ctx->p, lds, s);
-                const bool ok = pl.ok && res_compiled(j.ctx->a.physics, j.ctx->p.L, j.phase, pl.ry);
+                const bool ok = pl.ok && res_compiled(j.ctx->fdoh, j.ctx->a.physics, j.ctx->p.L, j.phase, pl.ry);
                 f.need[s] = ok && pl.tiles() <= ncu ? pl.tiles() : 0;
                 if (f.need[s] && (!f.least || f.need[s] < f.least)) f.least = f.need[s];
             }

@@ -50,7 +50,7 @@ struct ResKernel {
 };
 
 // is there a compiled kernel for this run (sw 0 forward, 1 adjoint) with ry rows per thread
-bool res_compiled(int physics, int L, int sw, int ry);
+bool res_compiled(int fdoh, int physics, int L, int sw, int ry);
 // enqueue one launch of as many workgroups, with the threads, LDS and thread
 // shape of pl; false when the runtime refuses it
 bool res_launch(const ResKernel &k, const ResPlan &pl, int blocks, int fdoh, int sw, void *stream);

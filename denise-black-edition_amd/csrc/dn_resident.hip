@@ -27,9 +27,9 @@ bool res_launch(const ResKernel &k, const ResPlan &pl, int blocks, int fdoh, int
     return false;
 }
 
-bool res_compiled(int physics, int L, int sw, int ry)
+bool res_compiled(int fdoh, int physics, int L, int sw, int ry)
 {
-    return physics >= 1 && physics <= 5 && (L == 0 || (physics == 1 && L <= 3)) && ry <= res_rows(L, sw);
+    return physics >= 1 && physics <= 5 && (L == 0 || (physics == 1 && L <= 3)) && ry <= res_rows(fdoh, physics, L, sw);
 }
 
 // ---------------------------------------------------------------- the pool

@@ -38,7 +38,7 @@ struct Cut {
             if (q.gx == 1 || p.nx - (q.gx - 1) * q.tw >= F) break;
         }
         // (a cell in both bands of an axis has two memory variables per derivative there)
-        if (ry > res_rows(p.L, 0) || p.ny < F || p.nx < 2 * p.fw || p.ny < 2 * p.fw) q.tw = 0;
+        if (ry > res_rows(F, phys, p.L, 0) || p.ny < F || p.nx < 2 * p.fw || p.ny < 2 * p.fw) q.tw = 0;
         q.nthx = q.tw / q.vx;
     }
     bool any() const { return q.tw >= 8; }

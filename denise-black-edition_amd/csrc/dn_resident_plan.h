@@ -22,14 +22,27 @@ constexpr int res_maxt(int ry, int vx, int F, int L)
 {
     return ry > 1 ? 512 : vx == 1 ? 1024 : vx == 2 ? (F <= 4 ? 1024 : 768) : (F <= 4 && L == 0 ? 768 : 512);
 }
-// Rows per thread, at most (sw: 0 forward, 1 adjoint).  Three relaxation
-// mechanisms (nine memory variables per cell) spill with several rows: the
-// sweeps were as fast or faster.  So do viscoelastic adjoint runs, and a trial
-// build of one with three mechanisms and two rows ended in a memory fault of
-// unknown cause: they take one-row shapes or the sweeps.  Two mechanisms,
-// forward: 2000x600 27 us a step against 31 in the sweeps, 1500x400 16
-// against 20.
-constexpr int res_rows(int L, int sw) { return L == 0 || (L < 3 && sw == 0) ? 3 : 1; }
+// Rows per thread, at most (ph: physics, sw: 0 forward, 1 adjoint).  Three
+// relaxation mechanisms (nine memory variables per cell) spill with several
+// rows: the sweeps were as fast or faster.  So do viscoelastic adjoint runs
+// (168 to 345 registers), and a trial build of one with three mechanisms and
+// two rows ended in a memory fault.  Its source keeps within bounds when it is
+// run on the host (tests/native/resident_exec.cpp), so the cause lies in what
+// was compiled and is not known: kernels with several rows that spill 100
+// registers or more are left out, but for the two of order 8 that are run and
+// tested (two mechanisms forward 159, TTI adjoint 136).  Without them: three
+// rows in elastic and VTI adjoint runs (103 to 153) and TTI forward runs (202,
+// 217) of orders 10 and 12, two and three rows in TTI adjoint runs of those (155 to 271), three
+// in TTI adjoint runs of order 6 (110) and in forward runs with two mechanisms
+// of the other orders (145 to 228).
+// Two mechanisms, forward, order 8: 2000x600 27 us a step against 31 in the
+// sweeps, 1500x400 16 against 20.
+constexpr int res_rows(int F, int ph, int L, int sw)
+{
+    if (L > 0) return L > 2 || sw ? 1 : L == 2 && F != 4 ? 2 : 3;
+    if (ph == 4) return F > 4 ? 2 - sw : F == 3 ? 3 - sw : 3;
+    return (ph == 1 || ph == 3) && F > 4 ? 3 - sw : 3;
+}
 constexpr int res_width(int ry) { return ry == 1 ? 32 : ry == 2 ? 64 : 72; }
 constexpr int RES_ENT = 256;     // sources and receivers of one tile and sweep kept in LDS, at most
 constexpr int res_ki(int F) { return F <= 4 ? 4 : 6; }  // halo words per thread and exchange, at most

@@ -450,7 +450,7 @@ void shape(const Grid &g, std::vector<float> &want)
     p.fdorder = 2 * CF;
     p.physics = CPH;
     p.L = CL;
-    if constexpr (RY <= res_rows(CL, CSW)) {
+    if constexpr (RY <= res_rows(CF, CPH, CL, CSW)) {
         const ResPlan least = res_least(p, 163840 - 2048, S);
         if (!least.ok) return;
         for (int more : {0, 5}) {

@@ -43,3 +43,25 @@ def test_no_flat_instructions(objects):
         text = subprocess.run([LLVM + "llvm-objdump", "-d", str(path)], capture_output=True, text=True, check=True).stdout
         assert "k_resident" in text and "global_load" in text
         assert "flat_" not in text
+
+
+def instances(objects):
+    """(half-order, rows, columns, pitch, physics, mechanisms, direction): vector registers spilled"""
+    out = {}
+    for path in objects:
+        notes = subprocess.run([LLVM + "llvm-readelf", "--notes", str(path)], capture_output=True, text=True,
+                               check=True).stdout
+        for block in notes.split("  - .agpr_count:")[1:]:
+            key = tuple(map(int, NAME.search(re.search(r"\.name:\s+(\S+)", block).group(1)).groups()))
+            out[key] = int(re.search(r"\.vgpr_spill_count:\s+(\d+)", block).group(1))
+    return out
+
+
+def test_spilled_registers(objects):
+    """No kernel with several rows per thread spills 100 registers or more,
+    but for the two of order 8 that the GPU tests run."""
+    got = instances(objects)
+    assert len({k[0] for k in got}) == 6 and len({(k[4], k[5], k[6]) for k in got}) == 16
+    heavy = {k: n for k, n in got.items() if k[1] > 1 and n >= 100}
+    assert set(heavy) <= {(4, 3, 4, 72, 1, 2, 0), (4, 3, 4, 72, 4, 0, 1)}, heavy
+    assert max(got.values()) < 168, max(got.items(), key=lambda kv: kv[1])
