@@ -528,6 +528,7 @@ ResArgs dn::res_args(const dn_ctx *c, const ResPlan &pl, const ResPoints &pt, co
     r.fwdstore = c->p.mode > 0;
     r.dtinv = c->p.dtinv > 0 ? c->p.dtinv : 1;
     r.vp1_form = c->p.grad_form == 1 || c->p.grad_form == 2;
+    r.spin = c->res_polls ? c->res_polls : RES_SPIN;
     r.rdh = 1.0 / (double)c->p.dh;
     const int v = 2 * sw, s = 2 * sw + 1;
     r.voff = lst + pt.off[v];
@@ -570,6 +571,12 @@ int res_run(dn_ctx *c, const StepCtl &ctl, int sw, int nsteps, bool *done)
     res_pool_give(c->res_pool, l);
     if (rc) return rc;
     *done = !aborted;
+    if (aborted) {
+        ++c->given_up;
+    } else {
+        c->ran_ry = pl.ry;
+        c->ran_vx = pl.vx;
+    }
     return DN_OK;
 }
 
@@ -1132,6 +1139,35 @@ int dn_get_tile(dn_ctx *c, int sweep, int *tbx, int *by, int *ty, int *vw)
     return DN_OK;
 }
 
+int dn_set_loop(dn_ctx *c, int rows, int cols, int polls)
+{
+    if (!c || polls < 0) return fail(DN_ERR_ARG, "bad loop request");
+    int shape = rows == 0 && cols == 0 ? -1 : RES_SHAPES;
+    for (int s = 0; s < RES_SHAPES; ++s)
+        if (res_shapes[s][0] == rows && res_shapes[s][1] == cols) shape = s;
+    if (shape == RES_SHAPES) return fail(DN_ERR_ARG, "no such thread shape");
+    if (!c->res_pool && shape >= 0) return fail(DN_ERR_STATE, "the device has no chip-resident loop");
+    HIP_OK(hipSetDevice(c->device));
+    HIP_OK(hipStreamSynchronize(c->stream));
+    ResPlan pl;
+    if (c->res_pool) pl = res_plan(c->p, res_pool_cus(c->res_pool), res_pool_lds(c->res_pool), shape);
+    if (shape >= 0 && !pl.ok) return fail(DN_ERR_ARG, "the grid does not fit this thread shape");
+    c->res = pl;
+    c->res_shape = shape;
+    c->res_polls = polls;
+    c->sweeps_chosen = false;
+    return build_lists(c);
+}
+
+int dn_get_loop(dn_ctx *c, int *rows, int *cols, int *given_up)
+{
+    if (!c) return fail(DN_ERR_ARG, "null context");
+    if (rows) *rows = c->ran_ry;
+    if (cols) *cols = c->ran_vx;
+    if (given_up) *given_up = c->given_up;
+    return DN_OK;
+}
+
 int dn_autotune_tile(dn_ctx *c, int nsteps, int *vel_shape, int *str_shape)
 {
     if (!c || nsteps < 1) return fail(DN_ERR_ARG, "autotune needs a context and nsteps >= 1");
@@ -1297,6 +1333,7 @@ int dn_run_forward(dn_ctx *c, int nsteps)
     if (c->eprecond)  // grad_obj_psv.c:71-76: the energies start at zero for each shot
         for (int w = 0; w < 2; ++w) HIP_OK(hipMemsetAsync(c->ew[w], 0, (size_t)c->p.nx * c->p.ny * sizeof(float), c->stream));
     HIP_OK(hipEventRecord(c->ev0, c->stream));
+    c->ran_ry = c->ran_vx = 0;
     if (res_applies(c, 0)) {
         bool done = false;
         if ((rc = res_run(c, ctl, 0, nsteps, &done))) return rc;
@@ -1454,6 +1491,7 @@ int dn_run_adjoint(dn_ctx *c, int nsteps)
     ctl.probe = 1;
     size_t nev = 0;
     HIP_OK(hipEventRecord(c->ev0, c->stream));
+    c->ran_ry = c->ran_vx = 0;
     if (res_applies(c, 1)) {
         bool done = false;
         if ((rc = res_run(c, ctl, 1, nsteps, &done)) || done) return rc;

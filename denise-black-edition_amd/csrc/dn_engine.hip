@@ -170,6 +170,7 @@ int plan_rounds(dn_engine *e)
         Fit f{k, 0, {}};
         if (!j.sweeps && res_applies(j.ctx, j.phase))
             for (int s = 0; s < RES_SHAPES; ++s) {
+                if (j.ctx->res_shape >= 0 && s != j.ctx->res_shape) continue;
                 const ResPlan pl = res_least(j.ctx->p, lds, s);
                 const bool ok = pl.ok && res_compiled(j.ctx->fdoh, j.ctx->a.physics, j.ctx->p.L, j.phase, pl.ry);
                 f.need[s] = ok && pl.tiles() <= ncu ? pl.tiles() : 0;
@@ -629,6 +630,11 @@ int dn_engine_launch(dn_engine *e, int nsteps)
     const bool changed = e->dirty || resident != e->resident;
     e->inflight = true;
     if (changed && (rc = rebuild(e, resident))) return rc;
+    for (const Job &j : e->jobs) {
+        const bool in = resident && j.round >= 0;
+        j.ctx->ran_ry = in ? j.plan.ry : 0;
+        j.ctx->ran_vx = in ? j.plan.vx : 0;
+    }
     if (resident && (rc = launch_rounds(e, left))) return rc;
     e->clock += left;
     // a graph is captured only for a set of shots that has already run
@@ -664,6 +670,8 @@ int dn_engine_wait(dn_engine *e, int *running)
                 HIP_OK(h2d(e->stream, e->d_clock + 1, word + 1, sizeof(int)));
                 for (Job &j : e->jobs) {
                     if (j.round < 0) continue;
+                    j.ctx->ran_ry = j.ctx->ran_vx = 0;
+                    ++j.ctx->given_up;
                     if ((rc = begin_shot(j.ctx, j.phase))) return rc;
                     j.sweeps = true;
                     j.base = e->clock - 1;

@@ -47,11 +47,12 @@ constexpr int res_width(int ry) { return ry == 1 ? 32 : ry == 2 ? 64 : 72; }
 constexpr int RES_ENT = 256;     // sources and receivers of one tile and sweep kept in LDS, at most
 constexpr int res_ki(int F) { return F <= 4 ? 4 : 6; }  // halo words per thread and exchange, at most
 constexpr int RES_CAP = 3072;                           // ... per tile and exchange
-// polls before a wait is given up: at the first exchange of a launch (its
-// workgroups may still wait for CUs that other work holds: about 20 ms) and
-// later (about a second; workgroups that answered once stay resident)
-constexpr int RES_SPIN_FIRST = 1 << 14;
+// polls before a wait is given up: later than the first exchange of a launch
+// (about a second; workgroups that answered once stay resident), and how many
+// powers of two fewer at the first (its workgroups may still wait for CUs
+// that other work holds: about 20 ms)
 constexpr int RES_SPIN = 1 << 20;
+constexpr int RES_SPIN_FIRST = 6;
 constexpr int RES_CHUNK = 2048;  // time steps per launch
 
 // the cut of a grid: gx x gy tiles of tw x th cells (tw a multiple of 4; the

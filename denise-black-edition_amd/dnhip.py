@@ -132,6 +132,8 @@ def load():
         "dn_set_snapshots": ([vp, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p], C.c_int),
         "dn_set_tile": ([vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int], C.c_int),
         "dn_get_tile": ([vp, C.c_int, ip, ip, ip, ip], C.c_int),
+        "dn_set_loop": ([vp, C.c_int, C.c_int, C.c_int], C.c_int),
+        "dn_get_loop": ([vp, ip, ip, ip], C.c_int),
         "dn_autotune_tile": ([vp, C.c_int, ip, ip], C.c_int),
         "dn_set_store_hint": ([vp, C.c_int, C.c_int], C.c_int),
         "dn_get_store_hint": ([vp, C.c_int, ip], C.c_int),
@@ -375,6 +377,18 @@ class Context:
         a, b, t, w = C.c_int(), C.c_int(), C.c_int(), C.c_int()
         _check(load().dn_get_tile(self.h, sweep, C.byref(a), C.byref(b), C.byref(t), C.byref(w)))
         return a.value, b.value, t.value, w.value
+
+    def set_loop(self, rows=0, cols=0, polls=0):
+        """Chip-resident loop: cells per thread (0, 0: the library's choice),
+        polls before a run is given up (0: the library's)."""
+        _check(load().dn_set_loop(self.h, rows, cols, polls))
+
+    def loop(self):
+        """Cells per thread of the last run (0, 0: it was the sweeps'), and
+        how many runs were given up and repeated by the sweeps."""
+        r, k, n = C.c_int(), C.c_int(), C.c_int()
+        _check(load().dn_get_loop(self.h, C.byref(r), C.byref(k), C.byref(n)))
+        return r.value, k.value, n.value
 
     def autotune(self, nsteps=50):
         """Pick the fastest compiled shape (tbx, by, ty, vw) of each sweep for
