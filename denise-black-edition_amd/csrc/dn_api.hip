@@ -573,7 +573,9 @@ int res_run(dn_ctx *c, const StepCtl &ctl, int sw, int nsteps, bool *done)
     *done = !aborted;
     if (aborted) {
         ++c->given_up;
+        c->res_rest.given_up();
     } else {
+        c->res_rest.finished();
         c->ran_ry = pl.ry;
         c->ran_vx = pl.vx;
     }
@@ -1155,6 +1157,7 @@ int dn_set_loop(dn_ctx *c, int rows, int cols, int polls)
     c->res = pl;
     c->res_shape = shape;
     c->res_polls = polls;
+    c->res_rest = ResRest();
     c->sweeps_chosen = false;
     return build_lists(c);
 }
@@ -1334,7 +1337,7 @@ int dn_run_forward(dn_ctx *c, int nsteps)
         for (int w = 0; w < 2; ++w) HIP_OK(hipMemsetAsync(c->ew[w], 0, (size_t)c->p.nx * c->p.ny * sizeof(float), c->stream));
     HIP_OK(hipEventRecord(c->ev0, c->stream));
     c->ran_ry = c->ran_vx = 0;
-    if (res_applies(c, 0)) {
+    if (res_applies(c, 0) && !c->res_rest.skip()) {
         bool done = false;
         if ((rc = res_run(c, ctl, 0, nsteps, &done))) return rc;
         if (done) {
@@ -1492,7 +1495,7 @@ int dn_run_adjoint(dn_ctx *c, int nsteps)
     size_t nev = 0;
     HIP_OK(hipEventRecord(c->ev0, c->stream));
     c->ran_ry = c->ran_vx = 0;
-    if (res_applies(c, 1)) {
+    if (res_applies(c, 1) && !c->res_rest.skip()) {
         bool done = false;
         if ((rc = res_run(c, ctl, 1, nsteps, &done)) || done) return rc;
         if ((rc = zero_state(c)) || (rc = zero_sums())) return rc;

@@ -93,6 +93,7 @@ struct dn_ctx {
     int *res_lst = nullptr;  // res_pts.blk on the device
     int res_shape = -1, res_polls = 0;      // dn_set_loop: entry of res_shapes, polls; -1, 0 the library's
     int ran_ry = 0, ran_vx = 0, given_up = 0;  // dn_get_loop
+    ResRest res_rest;
     // timing
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double run_ms = 0.0, v_ms = 0.0, s_ms = 0.0;

@@ -38,7 +38,7 @@ struct Job {
     dn_ctx *ctx;
     int phase;  // 0 forward, 1 adjoint
     long base;  // engine clock before its first step
-    bool sweeps = false;  // its chip-resident run was abandoned
+    bool sweeps = false;  // its chip-resident run was abandoned, or one before it
     int round = -1;       // the round that carries it, -1: the sweeps
     ResPlan plan;
     ResPoints pts;
@@ -102,6 +102,7 @@ struct dn_engine {
     std::vector<Round> rounds;
     bool resident = false;  // the sweeps' tables leave the shots of the rounds out
     bool leased = false;    // a launched run holds mailboxes and CUs
+    ResRest rest;           // shots attached after a given-up run
     ResLease lease;
     int *d_lst = nullptr;  // point lists
     ResBlock *d_rblk = nullptr;
@@ -593,6 +594,7 @@ int dn_engine_attach(dn_engine *e, dn_ctx *c, int phase)
     j.ctx = c;
     j.phase = phase;
     j.base = e->clock - 1;
+    j.sweeps = e->rest.skip();
     e->jobs.push_back(j);
     e->status[c] = 1;
     e->dirty = true;
@@ -663,7 +665,10 @@ int dn_engine_wait(dn_engine *e, int *running)
             e->leased = false;
             int word[2] = {0, 0};
             HIP_OK(d2h(e->stream, word, e->d_clock, sizeof word));
-            if (word[1]) {
+            if (!word[1]) {
+                e->rest.finished();
+            } else {
+                e->rest.given_up();
                 // the workgroups gave up waiting for each other: the shots of
                 // the rounds start over, in the sweeps
                 word[1] = 0;

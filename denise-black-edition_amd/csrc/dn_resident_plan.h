@@ -55,6 +55,26 @@ constexpr int RES_SPIN = 1 << 20;
 constexpr int RES_SPIN_FIRST = 6;
 constexpr int RES_CHUNK = 2048;  // time steps per launch
 
+// A run that was given up cost its waits, 20 ms and more, and the next one
+// would too while other work (another process's loop) holds the CUs: after
+// the k-th in a row, 2^k runs, 64 at most, take the sweeps before another try.
+struct ResRest {
+    int row = 0, left = 0;
+    // is this run one of those
+    bool skip()
+    {
+        if (left == 0) return false;
+        --left;
+        return true;
+    }
+    void given_up()
+    {
+        if (row < 6) ++row;
+        left = 1 << row;
+    }
+    void finished() { row = 0; }
+};
+
 // the cut of a grid: gx x gy tiles of tw x th cells (tw a multiple of 4; the
 // last ones of a row or column may be smaller), nthx x (th / ry) threads owning vx x ry
 // cells each, nthr threads in all

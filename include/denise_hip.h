@@ -244,7 +244,9 @@ int dn_get_tile(dn_ctx *ctx, int sweep, int *tbx, int *by, int *ty, int *vw);
  * dn_set_store_hint.  polls: how often a workgroup asks for its neighbours'
  * cells before the run is given up and repeated by the sweeps (it may wait
  * for CUs that other work holds); 0: about 20 ms at the start of a launch
- * and a second later.  DN_ERR_ARG where the grid does not fit the shape.
+ * and a second later.  After a run that was given up the next two take the
+ * sweeps at once, after a second in a row four, and so on to 64 (an engine
+ * counts its shots); dn_set_loop forgets them.  DN_ERR_ARG where the grid does not fit the shape.
  * dn_get_loop: cells per thread of the last run, 0 and 0 where it was the
  * sweeps', and how many runs of the context were given up; shots of an
  * engine count as runs.  Results do not depend on any of it.  No reference

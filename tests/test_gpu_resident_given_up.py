@@ -97,3 +97,34 @@ def test_engine_restarts_the_shots_of_its_rounds(first, beside):
         ref.forward()
         assert np.abs(ref.field(dnhip.F_VX)).max() > 0
         same(state(g, case[0]), state(ref, case[0]))
+
+
+def test_runs_after_a_given_up_one():
+    """The runs after it take the sweeps at once, two, four and so on, and the
+    loop is back when it is set anew."""
+    case = make_case(nx=200, ny=90, nt=30, fw=10)
+    g = context(case, False)
+    g.set_loop(polls=1)
+    tries = []
+    for _ in range(20):
+        g.forward()
+        tries.append(g.loop()[2])
+    assert tries == [1] * 3 + [2] * 5 + [3] * 9 + [4] * 3
+    g.set_loop()
+    g.forward()
+    assert g.loop() == (1, 1, 4)
+
+
+def test_shots_attached_after_a_given_up_run():
+    case = make_case(nx=200, ny=90, nt=30, fw=10)
+    eng = dnhip.Engine()
+    g = context(case, False)
+    paths = []
+    for polls in (1, 0, 0, 0):
+        g.set_loop(polls=polls)
+        eng.attach(g)
+        eng.step(30)
+        paths.append(g.loop()[0])
+        eng.run()
+        assert eng.status(g) == 0
+    assert paths == [0, 0, 0, 1] and g.loop()[2] == 1
