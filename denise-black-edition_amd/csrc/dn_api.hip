@@ -564,7 +564,7 @@ int res_run(dn_ctx *c, const StepCtl &ctl, int sw, int nsteps, bool *done)
         k.r.n1 = std::min(n + RES_CHUNK - 1, nsteps);
         k.r.tag0 = tag;
         tag += (unsigned)(k.r.n1 - k.r.n0 + 2);
-        ok = res_launch(k, pl, pl.tiles(), c->fdoh, sw, c->stream);
+        ok = res_launch(k, pl, pl.tiles(), c->fdoh, sw, res_pool_lds(c->res_pool), c->stream);
     }
     bool aborted = !ok;
     const int rc = finish_run(c, 0, &aborted);

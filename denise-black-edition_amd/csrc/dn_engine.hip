@@ -313,7 +313,7 @@ int launch_rounds(dn_engine *e, int steps)
             ResKernel k = tab[at];
             k.tab = e->d_rtab + at - slot;
             k.blk = e->d_rblk + r.blk;
-            if (!res_launch(k, r.shape, r.tiles, r.fdoh, r.sw, e->stream)) {
+            if (!res_launch(k, r.shape, r.tiles, r.fdoh, r.sw, res_pool_lds(e->pool), e->stream)) {
                 // the rounds already launched run to their end: every shot of
                 // the rounds starts over, as after an abandoned wait
                 static const int one = 1;

@@ -53,8 +53,9 @@ struct ResKernel {
 // is there a compiled kernel for this run (sw 0 forward, 1 adjoint) with ry rows per thread
 bool res_compiled(int fdoh, int physics, int L, int sw, int ry);
 // enqueue one launch of as many workgroups, with the threads, LDS and thread
-// shape of pl; false when the runtime refuses it
-bool res_launch(const ResKernel &k, const ResPlan &pl, int blocks, int fdoh, int sw, void *stream);
+// shape of pl on a device with lds_max bytes of LDS per workgroup; false when
+// the runtime refuses it
+bool res_launch(const ResKernel &k, const ResPlan &pl, int blocks, int fdoh, int sw, size_t lds_max, void *stream);
 
 // The mailboxes of a device: one allocation shared by the contexts on it,
 // made with the first and given back with the last, and the account of its

@@ -10,16 +10,16 @@
 namespace dn {
 
 template <int F, int GROUP>
-bool res_launch_f(const ResKernel &k, const ResPlan &pl, int blocks, int sw, hipStream_t s);
+bool res_launch_f(const ResKernel &k, const ResPlan &pl, int blocks, int sw, size_t lds_max, hipStream_t s);
 
-bool res_launch(const ResKernel &k, const ResPlan &pl, int blocks, int fdoh, int sw, void *stream)
+bool res_launch(const ResKernel &k, const ResPlan &pl, int blocks, int fdoh, int sw, size_t lds_max, void *stream)
 {
     hipStream_t s = (hipStream_t)stream;
 #define DN_F(F)                                                                \
     case F:                                                                    \
-        return k.a.physics != 1 ? res_launch_f<F, 1>(k, pl, blocks, sw, s) \
-               : k.a.L > 0      ? res_launch_f<F, 2>(k, pl, blocks, sw, s) \
-                                : res_launch_f<F, 0>(k, pl, blocks, sw, s);
+        return k.a.physics != 1 ? res_launch_f<F, 1>(k, pl, blocks, sw, lds_max, s) \
+               : k.a.L > 0      ? res_launch_f<F, 2>(k, pl, blocks, sw, lds_max, s) \
+                                : res_launch_f<F, 0>(k, pl, blocks, sw, lds_max, s);
     switch (fdoh) {
         DN_F(1) DN_F(2) DN_F(3) DN_F(4) DN_F(5) DN_F(6)
     }

@@ -112,3 +112,31 @@ def test_engine_rounds_of_every_shape(shape):
         assert np.abs(ref.gradient(0)).max() > 0
         for w in range(3):
             np.testing.assert_array_equal(g.gradient(w), ref.gradient(w), err_msg=f"{case[0].nx} sum {w}")
+
+
+def test_threads_share_a_kernel():
+    """Two contexts in two threads launch one kernel with different amounts of
+    LDS, and each launch is accepted."""
+    import threading
+    ctx = []
+    for nx, ny, nt in [(60, 30, 20), (1400, 480, 20)]:
+        case = make_case(nx=nx, ny=ny, nt=nt, fdorder=8, fw=10, homogeneous=True)
+        g = context(case, False)
+        g.set_loop(3, 4)
+        g.forward()
+        assert g.loop() == (3, 4, 0)
+        ctx.append(g)
+    paths = [set(), set()]
+
+    def work(k, n):
+        for _ in range(n):
+            ctx[k].forward()
+            paths[k].add(ctx[k].loop())
+
+    print("two threads, one kernel", flush=True)
+    ts = [threading.Thread(target=work, args=a) for a in [(0, 300), (1, 100)]]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert paths == [{(3, 4, 0)}] * 2
