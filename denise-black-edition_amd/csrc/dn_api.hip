@@ -653,6 +653,24 @@ std::vector<size_t> plan_sizes(const dn_params &p, int nsrc, int ntr)
     }
     return v;
 }
+
+// the cell lists beside them (build_lists, at the default tile shape): as
+// they are made with the context, and as its sources and receivers replace
+// them, since what those need may not fit into the blocks they leave
+std::vector<size_t> list_sizes(const dn_params &p, int nsrc, int ntr)
+{
+    const Tile t = default_tile(p.nx, p.ny);
+    const size_t ntiles = (size_t)t.ntx(p.nx) * t.nty(p.ny), loop_tiles = 256;
+    std::vector<size_t> v;
+    for (const size_t n : {(size_t)0, (size_t)nsrc + ntr}) {
+        for (int w = 0; w < 4; ++w) {
+            v.push_back((3 * ntiles + 1 + std::min(n, ntiles) * (t.width() + 1)) * sizeof(int));
+            v.push_back((n + 1) * sizeof(Ent));
+        }
+        v.push_back(4 * (loop_tiles + 2 + 3 * n) * sizeof(int));
+    }
+    return v;
+}
 }  // namespace dn
 
 extern "C" {

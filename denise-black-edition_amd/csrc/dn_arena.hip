@@ -10,6 +10,7 @@
 namespace dn {
 // device buffers a context with these parameters allocates (plan order)
 std::vector<size_t> plan_sizes(const dn_params &p, int nsrc, int ntr);
+std::vector<size_t> list_sizes(const dn_params &p, int nsrc, int ntr);
 }  // namespace dn
 
 int dn_arena_create(int device, size_t bytes, dn_arena **out)
@@ -60,8 +61,7 @@ int dn_arena_fits(dn_arena *a, const dn_params *p, int nsrc, int ntr, int *fits)
 {
     if (!a || !p || !fits || nsrc < 0 || ntr < 0) return fail(DN_ERR_ARG, "bad fit request");
     std::vector<size_t> sizes = plan_sizes(*p, nsrc, ntr);
-    // the cell lists of the four sweeps (a few bytes per point and tile)
-    for (int k = 0; k < 8; ++k) sizes.push_back(64 * 1024);
+    for (size_t n : list_sizes(*p, nsrc, ntr)) sizes.push_back(n);
     std::sort(sizes.rbegin(), sizes.rend());
     *fits = a->fits(sizes) ? 1 : 0;
     return DN_OK;

@@ -581,7 +581,9 @@ static void batch_init(run *r)
     dn_ok(dn_device_memory(0, &fr, &tot), "device memory");
     int ntest = 0;
     for (int ishot = 1; ishot <= r->nshots; ishot++) ntest += is_test_shot(r->P, ishot);
-    const size_t slack = 1 << 20; /* cell lists and alignment */
+    /* alignment and cell lists as dn_arena_fits counts them: some 0.4 bytes a
+     * cell and 1.2 kB a point */
+    const size_t slack = (1 << 20) + (size_t)p.nx * p.ny / 2 + (size_t)1536 * (r->nsrc + r->ntr);
     size_t need = (size_t)r->nshots * (fp + slack) + (size_t)ntest * (fp0 + slack);
     const size_t reserve = (size_t)4 << 30;
     size_t cap = fr > reserve ? (fr - reserve) / 10 * 9 : 0;

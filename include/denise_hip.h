@@ -311,7 +311,9 @@ int dn_device_memory(int device, size_t *free_bytes, size_t *total_bytes);
 /* Device bytes a context with these parameters, nsrc sources and ntr
  * receivers will hold (wavefields, material, CPML, seismograms and, for
  * params.mode > 0, the forward snapshots), computed without a device: the
- * admission test of a scheduler that packs shots into HBM. */
+ * admission test of a scheduler that packs shots into HBM.  Not counted: the
+ * cell lists (half a byte per cell, a kilobyte per point, at most) and the 12.6 MB
+ * of mailboxes that all contexts and engines of a device share. */
 int dn_estimate_footprint(const dn_params *p, int nsrc, int ntr, size_t *bytes);
 
 /* ---- Device-memory arena ---------------------------------------------------
