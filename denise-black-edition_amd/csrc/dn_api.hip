@@ -409,6 +409,7 @@ int validate(const dn_params *p)
 int dn::zero_state(dn_ctx *c)
 {
     ZeroList z;
+    static_assert(F_N + 3 + 9 + 1 <= ZeroList::MAX, "planes, memory variables, CPML arrays and the NaN word");
     const size_t pl = c->lay.plane();
     for (int k = 0; k < F_N; ++k)
         if (c->fld[k]) z.add(c->fld[k], pl);
