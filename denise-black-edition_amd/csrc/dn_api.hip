@@ -1038,6 +1038,14 @@ int dn_set_sources(dn_ctx *c, int nsrc, const float *srcpos, const float *signal
         drop(&q.src_ix), drop(&q.src_iy), drop(&q.src_type), drop(&q.src_sin), drop(&q.src_cos), drop(&q.signals);
         return build_lists(c);
     }
+    // a refused call leaves no sources: the cell lists must not name those of
+    // the call before, whose buffers may be gone
+    auto refuse = [&](int code) {
+        c->qtype = 0;
+        c->has_force = 0;
+        (void)build_lists(c);
+        return code;
+    };
     std::vector<int> ix(nsrc), iy(nsrc), type(nsrc);
     std::vector<double> sn(nsrc), cs(nsrc);
     for (int l = 0; l < nsrc; ++l) {
@@ -1049,8 +1057,8 @@ int dn_set_sources(dn_ctx *c, int nsrc, const float *srcpos, const float *signal
         sn[l] = std::sin((double)azi);
         cs[l] = std::cos((double)azi);
         if (ix[l] < 1 || ix[l] > c->p.nx || iy[l] < 1 || iy[l] > c->p.ny)
-            return fail(DN_ERR_ARG, "source " + std::to_string(l + 1) + " lies outside the grid");
-        if (type[l] == 5 && (ix[l] < 2 || iy[l] < 1)) return fail(DN_ERR_ARG, "moment-tensor source on the left edge");
+            return refuse(fail(DN_ERR_ARG, "source " + std::to_string(l + 1) + " lies outside the grid"));
+        if (type[l] == 5 && (ix[l] < 2 || iy[l] < 1)) return refuse(fail(DN_ERR_ARG, "moment-tensor source on the left edge"));
         if (type[l] >= 2 && type[l] <= 4) c->has_force = 1;
     }
     c->qtype = type[nsrc - 1];
@@ -1063,7 +1071,7 @@ int dn_set_sources(dn_ctx *c, int nsrc, const float *srcpos, const float *signal
         (rc = c->resize((void **)&q.src_sin, sizeof(double) * nsrc)) ||
         (rc = c->resize((void **)&q.src_cos, sizeof(double) * nsrc)) ||
         (rc = c->resize((void **)&q.signals, sizeof(float) * (size_t)nsrc * c->p.nt)))
-        return rc;
+        return refuse(rc);
     const Settle settle{c->stream};
     auto send = [&](void *to, const void *from, size_t n) {
         return hipMemcpyAsync(to, from, n, hipMemcpyHostToDevice, c->stream);
@@ -1110,15 +1118,22 @@ int dn_set_receivers(dn_ctx *c, int ntr, const int *recpos)
     c->rec_iy.assign(recpos + ntr, recpos + 2 * ntr);
     if (ntr == 0) return build_lists(c);
     const size_t tr = (size_t)ntr * c->p.nt * sizeof(float);
+    // (no memory: no receivers, likewise)
+    auto refuse = [&](int code) {
+        c->rec_ix.clear();
+        c->rec_iy.clear();
+        (void)build_lists(c);
+        return code;
+    };
     int rc;
     if ((rc = c->dalloc((void **)&q.rec_ix, sizeof(int) * ntr)) || (rc = c->dalloc((void **)&q.rec_iy, sizeof(int) * ntr)) ||
         (rc = c->dalloc((void **)&q.rec_sqlam, sizeof(double) * ntr)) ||
         (rc = c->dalloc((void **)&q.rec_sqmu, sizeof(double) * ntr)) || (rc = c->dalloc((void **)&q.obs, tr)))
-        return rc;
+        return refuse(rc);
     for (int k = 0; k < 5; ++k)
-        if ((rc = c->dalloc((void **)&q.sec[k], tr))) return rc;
+        if ((rc = c->dalloc((void **)&q.sec[k], tr))) return refuse(rc);
     for (int k = 0; k < 3; ++k)
-        if ((rc = c->dalloc((void **)&q.adj[k], tr))) return rc;
+        if ((rc = c->dalloc((void **)&q.adj[k], tr))) return refuse(rc);
     HIP_OK(h2d(c->stream, q.rec_ix, c->rec_ix.data(), sizeof(int) * ntr));
     HIP_OK(h2d(c->stream, q.rec_iy, c->rec_iy.data(), sizeof(int) * ntr));
     q.ntr = ntr;
