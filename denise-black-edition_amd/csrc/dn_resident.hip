@@ -55,7 +55,7 @@ bool clear(ResPool *p)
 {
     hipStream_t s = nullptr;
     const bool ok = hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess &&
-                    hipMemsetAsync(p->mem, 0, (p->words + 1024) * sizeof(res_word), s) == hipSuccess &&
+                    hipMemsetAsync(p->mem, 0, p->words * sizeof(res_word), s) == hipSuccess &&
                     hipStreamSynchronize(s) == hipSuccess;
     if (s) (void)hipStreamDestroy(s);
     if (ok)
@@ -86,9 +86,8 @@ ResPool *res_pool_open(int device)
     q->device = device;
     q->ncu = ncu;
     q->lds = (size_t)lds;
-    // (a workgroup reads past its last words, at most a word per thread)
     q->words = (size_t)ncu * 2 * RES_CAP;
-    if (hipMalloc((void **)&q->mem, (q->words + 1024) * sizeof(res_word)) != hipSuccess || !clear(q)) {
+    if (hipMalloc((void **)&q->mem, q->words * sizeof(res_word)) != hipSuccess || !clear(q)) {
         (void)hipGetLastError();
         if (q->mem) (void)hipFree(q->mem);
         delete q;

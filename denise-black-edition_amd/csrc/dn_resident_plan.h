@@ -16,8 +16,13 @@ namespace dn {
 
 // A thread owns RY rows of VX columns: 1 x 1, 1 x 2 or 1 x 4 in tiles up to
 // 32 columns wide, 2 x 4 or 3 x 4 in tiles up to 64 or 72 wide; the
-// widest tile fixes the LDS pitch at compile time.  A workgroup has as many threads as
-// the registers of that shape allow without spilling.
+// widest tile fixes the LDS pitch at compile time.  A workgroup has at most as
+// many threads as leave each the registers its shape asks for.  1 x 2 at
+// orders up to 8 has more: 128 registers, of which it spills up to 153 (elastic
+// order 8 55 forward, 115 adjoint), and more waves still win over more columns.  1000x400,
+// order 8, forward and adjoint steps with 1 x 2: 6.7 and 7.9 us, with 1 x 4 8.2
+// and 9.8; one mechanism 7.7, 8.9 and 8.6, 9.8; two 8.3, 10.0 and 9.2, 10.1; three
+// 9.7, 11.5 and 9.6, 10.4.
 constexpr int res_maxt(int ry, int vx, int F, int L)
 {
     return ry > 1 ? 512 : vx == 1 ? 1024 : vx == 2 ? (F <= 4 ? 1024 : 768) : (F <= 4 && L == 0 ? 768 : 512);
@@ -91,7 +96,8 @@ struct ResPlan {
 inline int res_planes(int physics) { return physics == 2 || physics == 5 ? 3 : 5; }
 
 // the plan of a grid on a device with ncu CUs and lds_max bytes of LDS per
-// workgroup (ok = false: the grid does not fit); shape: one entry of
+// workgroup (ok = false: the grid does not fit, in tiles as wide as the shape
+// allows); shape: one entry of
 // res_shapes, or -1 for the lightest that fits
 ResPlan res_plan(const dn_params &p, int ncu, size_t lds_max, int shape = -1);
 // the plan of that shape with the fewest tiles

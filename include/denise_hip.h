@@ -233,7 +233,8 @@ int dn_get_hc(dn_ctx *ctx, float *out7);
  * (128,2,2,2), (64,4,2,2); VTI/TTI stress sweeps take vw = 1 only.
  * Results do not depend on the shapes.  A context whose caller chose a shape
  * runs the sweeps; others run in the chip-resident time loop where their grid
- * fits it (up to about 1.3 million elastic cells).  No reference
+ * fits it (order 8, elastic: up to 1.02 million cells at least, 1.3 million at
+ * most; acoustic and SH 1.36 and 1.54).  No reference
  * counterpart: the reference has no GPU launch shapes. */
 int dn_set_tile(dn_ctx *ctx, int sweep, int tbx, int by, int ty, int vw);
 int dn_get_tile(dn_ctx *ctx, int sweep, int *tbx, int *by, int *ty, int *vw);
