@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -529,7 +530,7 @@ ResArgs dn::res_args(const dn_ctx *c, const ResPlan &pl, const ResPoints &pt, co
     r.fwdstore = c->p.mode > 0;
     r.dtinv = c->p.dtinv > 0 ? c->p.dtinv : 1;
     r.vp1_form = c->p.grad_form == 1 || c->p.grad_form == 2;
-    r.spin = c->res_polls ? c->res_polls : RES_SPIN;
+    r.quit = c->res_quit > 0 ? c->res_quit : INT_MAX;
     r.rdh = 1.0 / (double)c->p.dh;
     const int v = 2 * sw, s = 2 * sw + 1;
     r.voff = lst + pt.off[v];
@@ -1175,9 +1176,9 @@ int dn_get_tile(dn_ctx *c, int sweep, int *tbx, int *by, int *ty, int *vw)
     return DN_OK;
 }
 
-int dn_set_loop(dn_ctx *c, int rows, int cols, int polls)
+int dn_set_loop(dn_ctx *c, int rows, int cols, int quit)
 {
-    if (!c || polls < 0) return fail(DN_ERR_ARG, "bad loop request");
+    if (!c || quit < 0) return fail(DN_ERR_ARG, "bad loop request");
     int shape = rows == 0 && cols == 0 ? -1 : RES_SHAPES;
     for (int s = 0; s < RES_SHAPES; ++s)
         if (res_shapes[s][0] == rows && res_shapes[s][1] == cols) shape = s;
@@ -1190,7 +1191,7 @@ int dn_set_loop(dn_ctx *c, int rows, int cols, int polls)
     if (shape >= 0 && !pl.ok) return fail(DN_ERR_ARG, "the grid does not fit this thread shape");
     c->res = pl;
     c->res_shape = shape;
-    c->res_polls = polls;
+    c->res_quit = quit;
     c->res_rest = ResRest();
     c->sweeps_chosen = false;
     return build_lists(c);

@@ -91,7 +91,7 @@ struct dn_ctx {
     bool sweeps_chosen = false;
     ResPoints res_pts;
     int *res_lst = nullptr;  // res_pts.blk on the device
-    int res_shape = -1, res_polls = 0;      // dn_set_loop: entry of res_shapes, polls; -1, 0 the library's
+    int res_shape = -1, res_quit = 0;  // dn_set_loop: entry of res_shapes (-1: the library's choice), steps
     int ran_ry = 0, ran_vx = 0, given_up = 0;  // dn_get_loop
     ResRest res_rest;
     // timing

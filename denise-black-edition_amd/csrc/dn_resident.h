@@ -15,7 +15,7 @@ struct ResArgs {
     int tw, th, gx, gy, nthx, ncomp, nk_s, nk_v, cap, ncx, ncy, nve, nse;
     int n0, n1, nlast;  // time steps of this launch, last step of the run
     int fwdstore, dtinv, vp1_form;
-    int spin;           // polls before a wait is given up (RES_SPIN)
+    int quit;           // last step before the first tile abandons the run (dn_set_loop)
     double rdh;         // 1 / DH
     unsigned tag0;
     res_word *mbox;

@@ -34,30 +34,30 @@ constexpr int res_maxt(int ry, int vx, int F, int L)
 // two rows ended in a memory fault.  Its source keeps within bounds when it is
 // run on the host (tests/native/resident_exec.cpp), so the cause lies in what
 // was compiled and is not known: kernels with several rows that spill 100
-// registers or more are left out, but for the two of order 8 that are run and
-// tested (two mechanisms forward 159, TTI adjoint 136).  Without them: three
-// rows in elastic and VTI adjoint runs (103 to 153) and TTI forward runs (202,
-// 217) of orders 10 and 12, two and three rows in TTI adjoint runs of those (155 to 271), three
-// in TTI adjoint runs of order 6 (110) and in forward runs with two mechanisms
-// of the other orders (145 to 228).
+// registers or more are left out, but for the two of order 8 that have long
+// been run and tested (two mechanisms forward 147, TTI adjoint 126).  Left out:
+// three rows in elastic and VTI adjoint runs (103 to 153 registers) and in TTI
+// forward runs (202, 217) of orders 10 and 12, two and three in TTI adjoint
+// runs of those (155 to 271), three in TTI adjoint runs of orders 2 to 6 (73,
+// 113, 110), three in forward runs with two mechanisms of all orders but 8
+// (145 to 228).
 // Two mechanisms, forward, order 8: 2000x600 27 us a step against 31 in the
 // sweeps, 1500x400 16 against 20.
 constexpr int res_rows(int F, int ph, int L, int sw)
 {
     if (L > 0) return L > 2 || sw ? 1 : L == 2 && F != 4 ? 2 : 3;
-    if (ph == 4) return F > 4 ? 2 - sw : F == 3 ? 3 - sw : 3;
+    if (ph == 4) return sw && F != 4 ? (F > 4 ? 1 : 2) : F > 4 ? 2 : 3;
     return (ph == 1 || ph == 3) && F > 4 ? 3 - sw : 3;
 }
 constexpr int res_width(int ry) { return ry == 1 ? 32 : ry == 2 ? 64 : 72; }
 constexpr int RES_ENT = 256;     // sources and receivers of one tile and sweep kept in LDS, at most
 constexpr int res_ki(int F) { return F <= 4 ? 4 : 6; }  // halo words per thread and exchange, at most
 constexpr int RES_CAP = 3072;                           // ... per tile and exchange
-// polls before a wait is given up: later than the first exchange of a launch
-// (about a second; workgroups that answered once stay resident), and how many
-// powers of two fewer at the first (its workgroups may still wait for CUs
-// that other work holds: about 20 ms)
+// polls before a wait is given up: at the first exchange of a launch (its
+// workgroups may still wait for CUs that other work holds: about 20 ms) and
+// later (about a second; workgroups that answered once stay resident)
+constexpr int RES_SPIN_FIRST = 1 << 14;
 constexpr int RES_SPIN = 1 << 20;
-constexpr int RES_SPIN_FIRST = 6;
 constexpr int RES_CHUNK = 2048;  // time steps per launch
 
 // A run that was given up cost its waits, 20 ms and more, and the next one

@@ -378,10 +378,10 @@ class Context:
         _check(load().dn_get_tile(self.h, sweep, C.byref(a), C.byref(b), C.byref(t), C.byref(w)))
         return a.value, b.value, t.value, w.value
 
-    def set_loop(self, rows=0, cols=0, polls=0):
+    def set_loop(self, rows=0, cols=0, quit=0):
         """Chip-resident loop: cells per thread (0, 0: the library's choice),
-        polls before a run is given up (0: the library's)."""
-        _check(load().dn_set_loop(self.h, rows, cols, polls))
+        steps after which runs are given up on purpose (0: never)."""
+        _check(load().dn_set_loop(self.h, rows, cols, quit))
 
     def loop(self):
         """Cells per thread of the last run (0, 0: it was the sweeps'), and

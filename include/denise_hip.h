@@ -242,17 +242,17 @@ int dn_get_tile(dn_ctx *ctx, int sweep, int *tbx, int *by, int *ty, int *vw);
 /* Chip-resident time loop.  dn_set_loop: cells per thread (rows, cols), one
  * of (1,1), (1,2), (1,4), (2,4), (3,4), or (0,0) for the lightest that fits
  * (the default); it takes back a choice of the sweeps by dn_set_tile or
- * dn_set_store_hint.  polls: how often a workgroup asks for its neighbours'
- * cells before the run is given up and repeated by the sweeps (it may wait
- * for CUs that other work holds); 0: about 20 ms at the start of a launch
- * and a second later.  After a run that was given up the next two take the
+ * dn_set_store_hint.  A run whose workgroups wait for each other too long
+ * (CUs that other work holds: 20 ms at the start of a launch, a second later)
+ * is given up and repeated by the sweeps; the next two runs then take the
  * sweeps at once, after a second in a row four, and so on to 64 (an engine
- * counts its shots); dn_set_loop forgets them.  DN_ERR_ARG where the grid does not fit the shape.
+ * counts its shots); dn_set_loop forgets them.  quit: steps after which runs
+ * are given up on purpose (up to 16 later), for tests; 0 never.  DN_ERR_ARG where the grid does not fit the shape.
  * dn_get_loop: cells per thread of the last run, 0 and 0 where it was the
  * sweeps', and how many runs of the context were given up; shots of an
  * engine count as runs.  Results do not depend on any of it.  No reference
  * counterpart. */
-int dn_set_loop(dn_ctx *ctx, int rows, int cols, int polls);
+int dn_set_loop(dn_ctx *ctx, int rows, int cols, int quit);
 int dn_get_loop(dn_ctx *ctx, int *rows, int *cols, int *given_up);
 
 /* Cache policy of a sweep: 0 plain; 1 streaming (nontemporal) loads of the

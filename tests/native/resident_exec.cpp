@@ -414,7 +414,7 @@ void advance(Shot &s, const ResPlan &plan, int cut)
     r.fwdstore = CSW == 0;
     r.dtinv = s.g.dtinv;
     r.vp1_form = 1;
-    r.spin = RES_SPIN;
+    r.quit = 1 << 30;
     r.rdh = 1.0 / (double)s.k.a.dh;
     std::unique_ptr<res_word[]> box(new res_word[(size_t)pl.tiles() * 2 * pl.cap]());
     r.mbox = box.get();

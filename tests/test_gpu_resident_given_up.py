@@ -1,7 +1,8 @@
-"""Runs of the chip-resident time loop whose workgroups give up waiting for
-each other (one poll a wait, dn_set_loop) leave partial states, snapshots and
-sums behind; the repeat by the sweeps has to discard them all.  Every kernel
-exits normally: the waits are bounded."""
+"""Runs of the chip-resident time loop that are given up leave partial states,
+snapshots and sums behind; the repeat by the sweeps has to discard them all.
+The workgroup of the first tile leaves after the steps that dn_set_loop gives,
+as after a wait that took too long; the others find its flag in their waits.
+Every kernel exits normally."""
 import numpy as np
 import pytest
 
@@ -40,7 +41,7 @@ def test_forward_and_adjoint_repeat(shape, L):
     print(f"given up: shape {shape} L {L}", flush=True)
     # the forward run given up; the adjoint run reads the repeat's snapshots
     g = context(case, False)
-    g.set_loop(*shape, polls=1)
+    g.set_loop(*shape, quit=20)
     g.forward()
     assert g.loop() == (0, 0, 1)
     same(state(g, p), fwd)
@@ -52,17 +53,19 @@ def test_forward_and_adjoint_repeat(shape, L):
     g.set_loop(*shape)
     g.forward()
     assert g.loop() == shape + (0,)
-    g.set_loop(*shape, polls=1)
+    g.set_loop(*shape, quit=20)
     same(adjoint(g, p), adj)
     assert g.loop() == (0, 0, 1)
     g.close()
 
 
-def test_run_of_several_launches_repeats():
+@pytest.mark.parametrize("quit", [20, 2040, 3000, 4200])
+def test_run_of_several_launches_repeats(quit):
+    """Given up in the first, second and third launch of 2048 steps."""
     case = make_case(nx=200, ny=90, nt=4500, fw=10)
     g, ref = context(case, False), context(case, True)
-    g.set_loop(polls=1)
-    print("given up: 4500 steps", flush=True)
+    g.set_loop(quit=quit)
+    print(f"given up: after {quit} of 4500 steps", flush=True)
     g.forward()
     assert g.loop() == (0, 0, 1)
     ref.forward()
@@ -87,7 +90,7 @@ def test_engine_restarts_the_shots_of_its_rounds(first, beside):
     if first:
         eng.step(first)
         assert [g.loop()[0] > 0 for g in shots] == [True, True, False][:len(shots)]
-    shots[1].set_loop(polls=1)
+    shots[1].set_loop(quit=first + 20)
     eng.step(40)
     assert [g.loop()[1:] for g in shots] == [(0, 1), (0, 1), (0, 0)][:len(shots)]
     eng.run()
@@ -104,7 +107,7 @@ def test_runs_after_a_given_up_one():
     loop is back when it is set anew."""
     case = make_case(nx=200, ny=90, nt=30, fw=10)
     g = context(case, False)
-    g.set_loop(polls=1)
+    g.set_loop(quit=10)
     tries = []
     for _ in range(20):
         g.forward()
@@ -120,8 +123,8 @@ def test_shots_attached_after_a_given_up_run():
     eng = dnhip.Engine()
     g = context(case, False)
     paths = []
-    for polls in (1, 0, 0, 0):
-        g.set_loop(polls=polls)
+    for quit in (10, 0, 0, 0):
+        g.set_loop(quit=quit)
         eng.attach(g)
         eng.step(30)
         paths.append(g.loop()[0])

@@ -18,7 +18,7 @@ def rows(fdorder, physics, L, adjoint):
     if L > 0:
         return 1 if L > 2 or adjoint else 2 if L == 2 and fdorder != 8 else 3
     if physics == 4:
-        return 2 - adjoint if fdorder > 8 else 3 - adjoint if fdorder == 6 else 3
+        return 3 if fdorder == 8 else (1 if fdorder > 8 else 2) if adjoint else 2 if fdorder > 8 else 3
     return 3 - adjoint if physics in (1, 3) and fdorder > 8 else 3
 
 
