@@ -571,7 +571,6 @@ int res_run(dn_ctx *c, const StepCtl &ctl, int sw, int nsteps, bool *done)
     bool aborted = !ok;
     const int rc = finish_run(c, 0, &aborted);
     res_pool_give(c->res_pool, l);
-    if (rc) return rc;
     *done = !aborted;
     if (aborted) {
         ++c->given_up;
@@ -581,7 +580,7 @@ int res_run(dn_ctx *c, const StepCtl &ctl, int sw, int nsteps, bool *done)
         c->ran_ry = pl.ry;
         c->ran_vx = pl.vx;
     }
-    return DN_OK;
+    return rc;
 }
 
 int receiver_factors(dn_ctx *c)

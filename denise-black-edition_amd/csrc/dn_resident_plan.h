@@ -18,11 +18,11 @@ namespace dn {
 // 32 columns wide, 2 x 4 or 3 x 4 in tiles up to 64 or 72 wide; the
 // widest tile fixes the LDS pitch at compile time.  A workgroup has at most as
 // many threads as leave each the registers its shape asks for.  1 x 2 at
-// orders up to 8 has more: 128 registers, of which it spills up to 153 (elastic
-// order 8 55 forward, 115 adjoint), and more waves still win over more columns.  1000x400,
-// order 8, forward and adjoint steps with 1 x 2: 6.7 and 7.9 us, with 1 x 4 8.2
-// and 9.8; one mechanism 7.7, 8.9 and 8.6, 9.8; two 8.3, 10.0 and 9.2, 10.1; three
-// 9.7, 11.5 and 9.6, 10.4.
+// orders up to 8 has more: 128 registers a thread, and it spills up to 133
+// (elastic, order 8, 23 forward and 97 adjoint).  More waves still win over
+// more columns: 1000x400, order 8, forward and adjoint steps 6.7 and 7.9 us with
+// 1 x 2, 8.2 and 9.8 with 1 x 4; one mechanism 7.7, 8.9 and 8.6, 9.8; two 8.3, 10.0
+// and 9.2, 10.1; with three they do not (9.7, 11.5 and 9.6, 10.4).
 constexpr int res_maxt(int ry, int vx, int F, int L)
 {
     return ry > 1 ? 512 : vx == 1 ? 1024 : vx == 2 ? (F <= 4 ? 1024 : 768) : (F <= 4 && L == 0 ? 768 : 512);
